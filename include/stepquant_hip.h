@@ -249,6 +249,32 @@ typedef struct sq_prefill_args {
 int sq_prefill(const sq_pool *pool, const sq_prefill_args *args, void *stream);
 
 /*
+ * The same prefill with long sequences cut into segments that run side by
+ * side, for calls whose sequences x heads leave most of the device idle (the
+ * recurrence is serial along a sequence).  sq_prefill_plan decides from the
+ * host copy of cu_seqlens and the compute units (`cus`; 0 or less: the
+ * current device's): tokens == 0 means whole sequences are the faster way
+ * (no workspace), otherwise segments of `tokens` tokens, at most `count` a
+ * sequence, and the device workspace they need.  The caller allocates it
+ * (16-byte aligned), sets `workspace` and hands the plan, with the same
+ * cu_seqlens, to sq_prefill_split; NULL or tokens == 0 there is sq_prefill.
+ * Three launches: every segment's effect on a state (S_end = M S_start + E,
+ * both fp32), the start states from them, the segments themselves.
+ * No counterpart in the reference.
+ */
+typedef struct sq_prefill_segments {
+    int32_t tokens;
+    int32_t count;
+    int64_t workspace_bytes;
+    void *workspace;
+} sq_prefill_segments;
+
+int sq_prefill_plan(const sq_pool *pool, const int32_t *cu_seqlens, int64_t batch, int32_t cus,
+                    sq_prefill_segments *segments);
+int sq_prefill_split(const sq_pool *pool, const sq_prefill_args *args, const sq_prefill_segments *segments,
+                     void *stream);
+
+/*
  * Slot operations (pool.py:358-365).  sq_clear_slots zeroes whole pages.
  * sq_copy_slots copies pages src[i] -> dst[i] through `temp`
  * ([n, page_bytes] bytes) so overlapping index sets behave like the

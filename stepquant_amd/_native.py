@@ -57,6 +57,11 @@ class PrefillArgs(ctypes.Structure):
                 ("beta_logits", ctypes.c_int32), ("reserved", ctypes.c_int32)]
 
 
+class PrefillSegments(ctypes.Structure):
+    _fields_ = [("tokens", ctypes.c_int32), ("count", ctypes.c_int32), ("workspace_bytes", ctypes.c_int64),
+                ("workspace", _P)]
+
+
 class FormatPool(ctypes.Structure):
     _fields_ = [("data", _P), ("page_bytes", ctypes.c_int64), ("num_slots", ctypes.c_int64),
                 ("offsets", _P), ("rows", _P), ("columns", _P), ("heads", ctypes.c_int32),
@@ -71,6 +76,7 @@ FMT_ROWS_CONTIGUOUS = 1
 EXPORTS = ("sq_abi_version", "sq_last_error", "sq_encode", "sq_decode_dense", "sq_decode_step",
            "sq_decode_readout", "sq_writeback", "sq_clear_slots", "sq_copy_slots",
            "sq_stream_capture_id", "sq_create_cu_stream", "sq_pool_flags", "sq_prefill",
+           "sq_prefill_plan", "sq_prefill_split",
            "sq_format_encode", "sq_format_decode", "sq_format_step", "sq_copy_slots_static",
            "sq_event_create", "sq_event_destroy", "sq_event_record", "sq_event_wait", "sq_event_query",
            "sq_event_synchronize")
@@ -101,6 +107,8 @@ def lib():
     L.sq_decode_readout.argtypes = [PP(Pool), PP(StepArgs), PP(Scratch), _P]
     L.sq_writeback.argtypes = [PP(Pool), PP(Scratch), ctypes.c_int64, _P]
     L.sq_prefill.argtypes = [PP(Pool), PP(PrefillArgs), _P]
+    L.sq_prefill_plan.argtypes = [PP(Pool), _P, ctypes.c_int64, ctypes.c_int32, PP(PrefillSegments)]
+    L.sq_prefill_split.argtypes = [PP(Pool), PP(PrefillArgs), PP(PrefillSegments), _P]
     L.sq_format_encode.argtypes = [PP(FormatPool), _P, _P, ctypes.c_int32, ctypes.c_int64, _P]
     L.sq_format_decode.argtypes = [PP(FormatPool), _P, ctypes.c_int32, ctypes.c_int64, _P, _P]
     L.sq_format_step.argtypes = [PP(FormatPool), PP(StepArgs), _P]
@@ -158,6 +166,13 @@ def pool_flags(bits, head_meta, columns, H, K, V, group, kda, storage, page_byte
     if rc < 0:
         check(rc, "pool flags")
     return rc
+
+
+def prefill_plan(pool: Pool, cu_seqlens: torch.Tensor, cus: int = 0) -> PrefillSegments:
+    """sq_prefill_plan of host int32 sequence offsets."""
+    segments = PrefillSegments()
+    check(lib().sq_prefill_plan(pool, cu_seqlens.data_ptr(), cu_seqlens.numel() - 1, cus, segments), "prefill plan")
+    return segments
 
 
 def capture_id(stream) -> int | None:

@@ -3390,7 +3390,32 @@ struct PrefillDev {
   float scale;
   int page_init;  // 1: initial states decoded from the pages of pi.slots inside the kernel
   PageInit pi;
+  // sequences cut into segments of seg tokens (0: whole sequences); seg_state
+  // and seg_trans hold [segment slot][H][K][V] f32 (see Segment)
+  int seg;
+  float *seg_state, *seg_trans;
 };
+
+// One segment of a sequence: tokens t0 .. t0 + len - 1 of the packed rows,
+// start tokens into its sequence.  Its workspace slot t0_seq / seg + b + s is
+// distinct for every (b, s): a sequence takes at most ceil(len / seg) slots
+// and the next one starts at least floor(len / seg) + 1 further.
+struct Segment {
+  int t0, len, start, slot;
+  bool last;  // of its sequence
+};
+__device__ __forceinline__ Segment segment_of(const PrefillDev &D, int b, int s) {
+  Segment r;
+  const int t0 = __builtin_amdgcn_readfirstlane(D.cu[b]);
+  const int len = __builtin_amdgcn_readfirstlane(D.cu[b + 1]) - t0;
+  if (D.seg == 0) return Segment{t0, len, 0, 0, true};
+  r.start = s * D.seg;
+  r.t0 = t0 + r.start;
+  r.len = len - r.start < D.seg ? len - r.start : D.seg;
+  r.slot = (int)((unsigned)t0 / (unsigned)D.seg) + b + s;
+  r.last = r.start + D.seg >= len;
+  return r;
+}
 
 // Element (r, t) of the transposed k tile sits in row r at column
 // tcol(r, t): the 8-token block index is XORed with bits 3-5 of r, so rows
@@ -3634,13 +3659,21 @@ __device__ __forceinline__ void init_from_page(const PageInit &pi, int b, int h,
   }
 }
 
-// One workgroup of 8 waves per (sequence, head), chunks in order.  Wave w
+// One workgroup of 8 waves per (sequence, head), chunks in order; with D.seg,
+// per (sequence segment, head), blockIdx.y the segment, whose start state the
+// combine kernel left in D.seg_state.  SUMMARY: no outputs, checkpoints or
+// queries, only what segment blockIdx.y does to a state, S_end = M S_start + E:
+// E from a start state of zero (segment 0: the true one), M from the identity
+// with v = 0 (each state column passes through the recurrence alone, so the
+// columns of M are its images of the unit vectors), both in one workgroup,
+// which stages the chunk and solves its A once.  Wave w
 // owns the 16 state columns j = 16 w .. 16 w + 15 for all 128 rows d (in
 // registers, accumulator layout); R, Delta and Delta' of its columns stay in
 // registers too and reach the next product through to_operand.  The chunk's
 // k, q, v, A, T and P are shared through LDS.  Transposed products keep every
 // operand in a layout it already has: O^T = S0^T Q^T + Delta^T P^T gives
 // each lane 4 consecutive output columns for one token.
+template <bool SUMMARY>
 __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
 #pragma clang fp contract(off)
   extern __shared__ __align__(16) uint8_t smem[];
@@ -3658,9 +3691,14 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
   const int b = x / H;
   const int hk = h / G;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, q4 = l >> 4, c16 = l & 15;
-  // sequence bounds as wave-uniform values (addresses formed from them stay scalar)
-  const int t0 = __builtin_amdgcn_readfirstlane(D.cu[b]), len = __builtin_amdgcn_readfirstlane(D.cu[b + 1]) - t0;
-  if (len <= 0) return;  // whole workgroup: an empty sequence has no chunk and no checkpoint
+  // segment bounds as wave-uniform values (addresses formed from them stay scalar)
+  const int seg_i = blockIdx.y;
+  const bool trans = SUMMARY && seg_i > 0;  // M wanted
+  const Segment sg = segment_of(D, b, seg_i);
+  const int t0 = sg.t0, len = sg.len;
+  // whole workgroup: an empty sequence has no chunk and no checkpoint; a
+  // sequence's last segment needs no summary and its first no M
+  if (len <= 0 || (SUMMARY && sg.last)) return;
   float *sm = (float *)(smem + OFF_SM);
   uint8_t *Kc = smem + OFF_KC, *Qc = smem + OFF_QC, *Kt = smem + OFF_KT, *Vc = smem + OFF_VC;
   float *AT = (float *)(smem + OFF_AT);
@@ -3681,19 +3719,32 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
   };
 
   // ---- state S[d][j] of this wave's columns: tile dt holds rows d = 16 dt + 4 q4 + r, column jw + c16
-  f32x4 S[8];
-  if (D.page_init) {
+  f32x4 S[8], M[SUMMARY ? 8 : 1];  // M: the same columns of the segment's M
+  if (SUMMARY) {
+#pragma unroll
+    for (int dt = 0; dt < (SUMMARY ? 8 : 0); dt++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        M[dt][r] = 16 * dt + 4 * q4 + r == jw + c16 ? 1.0f : 0.0f;
+        S[dt][r] = 0.0f;
+      }
+  }
+  if (SUMMARY && seg_i > 0) {
+    // E from zero
+  } else if (D.page_init && seg_i == 0) {
     init_from_page(D.pi, b, h, smem, tid, S);
     __syncthreads();  // the staged page is read before the first chunk's tiles overwrite it
   } else {
-    const float *src = D.init + ((int64_t)b * H + h) * PKD * PV + jw + c16;
+    // the sequence's dense initial state, or the segment's start state
+    const float *src = (seg_i == 0 ? D.init + ((int64_t)b * H + h) * PKD * PV
+                                   : D.seg_state + ((int64_t)(sg.slot - 1) * H + h) * PKD * PV) + jw + c16;
 #pragma unroll
     for (int dt = 0; dt < 8; dt++)
 #pragma unroll
       for (int r = 0; r < 4; r++) S[dt][r] = src[(int64_t)(16 * dt + 4 * q4 + r) * PV];
   }
-  // this sequence's checkpoints (ascending), one per lane
-  const int ckv = l < D.NC ? D.ckpt[(int64_t)b * D.NC + l] : 0x7fffffff;
+  // this sequence's checkpoints (ascending) past the segment's start, one per lane
+  const int ckv = !SUMMARY && l < D.NC ? D.ckpt[(int64_t)b * D.NC + l] - sg.start : 0x7fffffff;
   // tokens of the segment starting at c: up to the first listed checkpoint
   // past c (within the sequence), the sequence end, or one chunk
   auto segment = [&](int c) {
@@ -3721,7 +3772,7 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
       const int idx = tid + NT * it, t = idx >> 4, d8 = (idx & 15) * 8;
       const uint32_t tr = (uint32_t)(t < lim ? t : lim), db = 2u * (uint32_t)d8;
       F.k[it] = *(const uint4 *)(kb + (__umul24(tr, 2u * (uint32_t)D.k_stride) + db));
-      F.q[it] = *(const uint4 *)(qb + (__umul24(tr, 2u * (uint32_t)D.q_stride) + db));
+      if (!SUMMARY) F.q[it] = *(const uint4 *)(qb + (__umul24(tr, 2u * (uint32_t)D.q_stride) + db));
       F.v[it] = *(const uint4 *)(vb + (__umul24(tr, 2u * (uint32_t)D.v_stride) + db));
     }
     if (w == 0) {
@@ -3757,12 +3808,15 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
     for (int it = 0; it < 2; it++) {
       const int idx = tid + NT * it, t = idx >> 4, d8 = (idx & 15) * 8;
       const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
-      const uint4 kv = t < n ? F.k[it] : zero, qv = t < n ? F.q[it] : zero, vv = t < n ? F.v[it] : zero;
+      const uint4 kv = t < n ? F.k[it] : zero, vv = t < n ? F.v[it] : zero;
+      const uint4 qv = !SUMMARY && t < n ? F.q[it] : zero;
       // key columns d8 .. d8 + 3 and d8 + 4 .. d8 + 7 at their permuted places
       *(uint2 *)(Kc + (t * P136 + pcol(d8)) * 2) = make_uint2(kv.x, kv.y);
       *(uint2 *)(Kc + (t * P136 + pcol(d8 + 4)) * 2) = make_uint2(kv.z, kv.w);
-      *(uint2 *)(Qc + (t * P136 + pcol(d8)) * 2) = make_uint2(qv.x, qv.y);
-      *(uint2 *)(Qc + (t * P136 + pcol(d8 + 4)) * 2) = make_uint2(qv.z, qv.w);
+      if (!SUMMARY) {
+        *(uint2 *)(Qc + (t * P136 + pcol(d8)) * 2) = make_uint2(qv.x, qv.y);
+        *(uint2 *)(Qc + (t * P136 + pcol(d8 + 4)) * 2) = make_uint2(qv.z, qv.w);
+      }
       *(uint4 *)(Vc + (t * P136 + d8) * 2) = vv;
       // squared norms of the 8 values, two bf16 products per v_dot2_f32_bf16
       float sk = 0.f, sq = 0.f;
@@ -3772,8 +3826,9 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
         for (int e = 0; e < 4; e++) {
           sk = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, kw[e]), __builtin_bit_cast(bf16x2, kw[e]),
                                                sk, false);
-          sq = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, qw[e]), __builtin_bit_cast(bf16x2, qw[e]),
-                                               sq, false);
+          if (!SUMMARY)
+            sq = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, qw[e]), __builtin_bit_cast(bf16x2, qw[e]),
+                                                 sq, false);
         }
       }
       {
@@ -3791,10 +3846,10 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
                                                    __builtin_amdgcn_perm(x[3], x[2], 0x07060302u));
       }
       sk = row16_sum(sk);
-      sq = row16_sum(sq);
+      if (!SUMMARY) sq = row16_sum(sq);
       if ((idx & 15) == 0) {
         sm[SM_KSQ * 64 + t] = sk;
-        sm[SM_QSQ * 64 + t] = sq;
+        if (!SUMMARY) sm[SM_QSQ * 64 + t] = sq;
       }
     }
     if (w == 0) {
@@ -3821,18 +3876,50 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
     if (tid < 64) {
       const int t = tid;
       const float nk = D.normalize ? __builtin_amdgcn_rsqf(sm[SM_KSQ * 64 + t] + 1e-6f) : 1.0f;
-      const float nq = (D.normalize ? __builtin_amdgcn_rsqf(sm[SM_QSQ * 64 + t] + 1e-6f) : 1.0f) * D.scale;
       const float lc = sm[SM_LC * 64 + t], lcC = sm[SM_LC * 64 + 63];
       const float gam = __expf(lc);
       sm[SM_NK * 64 + t] = nk;
-      sm[SM_NQ * 64 + t] = nq;
       sm[SM_GK * 64 + t] = gam * nk;  // Gamma_t nk_t
-      sm[SM_QG * 64 + t] = nq * gam;
+      if (!SUMMARY) {
+        const float nq = (D.normalize ? __builtin_amdgcn_rsqf(sm[SM_QSQ * 64 + t] + 1e-6f) : 1.0f) * D.scale;
+        sm[SM_NQ * 64 + t] = nq;
+        sm[SM_QG * 64 + t] = nq * gam;
+      }
       sm[SM_KD * 64 + t] = nk * __expf(lcC - lc);
     }
     lds_barrier();
 
     f32x4 R[4], oq[4];
+    // R = beta (V - Gamma nk K S0) of this wave's columns (with_v false: V = 0);
+    // key-slot blocks outermost: the four token tiles' accumulators are
+    // independent, so each block's loads are in flight while the previous
+    // block's products run
+    auto ks_of = [&](const bf16x8 (&sh)[4], const bf16x8 (&sl)[4], f32x4 (&R)[4], bool with_v) {
+      f32x4 ak[4];
+#pragma unroll
+      for (int tt = 0; tt < 4; tt++) ak[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kc = 0; kc < 4; kc++) {
+        bf16x8 kr[4];
+#pragma unroll
+        for (int tt = 0; tt < 4; tt++) kr[tt] = ld8(Kc, ((16 * tt + c16) * P136 + 32 * kc + 8 * q4) * 2);
+#pragma unroll
+        for (int tt = 0; tt < 4; tt++) ak[tt] = mfma(kr[tt], sh[kc], ak[tt]);
+#pragma unroll
+        for (int tt = 0; tt < 4; tt++) ak[tt] = mfma(kr[tt], sl[kc], ak[tt]);
+      }
+#pragma unroll
+      for (int tt = 0; tt < 4; tt++) {
+        const int ta = 16 * tt + 4 * q4;
+        const float4 be = *(const float4 *)(sm + SM_BETA * 64 + ta), gk = *(const float4 *)(sm + SM_GK * 64 + ta);
+        const float be4[4] = {be.x, be.y, be.z, be.w}, gk4[4] = {gk.x, gk.y, gk.z, gk.w};
+        const tr4_t vr = col4(Vc, ta, jw, c16);  // v of tokens ta .. ta + 3, column jw + c16
+        const float v4[4] = {bf2f((uint16_t)vr[0]), bf2f((uint16_t)vr[1]), bf2f((uint16_t)vr[2]),
+                             bf2f((uint16_t)vr[3])};
+#pragma unroll
+        for (int r = 0; r < 4; r++) R[tt][r] = be4[r] * ((with_v ? v4[r] : 0.0f) - gk4[r] * ak[tt][r]);
+      }
+    };
     // ---- A and P tiles (t-tile tw, s-tile ns) with ns <= tw:
     // A_ts = beta_t nk_t nk_s (Gamma_t/Gamma_s) k_t.k_s (s < t), P_ts likewise with q_t (s <= t).
     // The ten tiles go at most two to a wave; tiles above the diagonal stay
@@ -3848,7 +3935,7 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
           if (doP) bq[ks] = ld8(Qc, (t * P136 + 8 * q4 + 32 * ks) * 2);
         }
         const float lct = sm[SM_LC * 64 + t], bnt = sm[SM_BETA * 64 + t] * sm[SM_NK * 64 + t];
-        const float nqt = sm[SM_NQ * 64 + t];
+        const float nqt = doP ? sm[SM_NQ * 64 + t] : 0.0f;
         f32x4 aA = {0.f, 0.f, 0.f, 0.f}, aP = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) {
@@ -3913,35 +4000,7 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
       bf16x8 sh[4], sl[4];
 #pragma unroll
       for (int kc = 0; kc < 4; kc++) split8(S[2 * kc], S[2 * kc + 1], sh[kc], sl[kc]);
-      // key-slot blocks outermost: the four token tiles' accumulators are
-      // independent, so each block's loads are in flight while the previous
-      // block's products run
-      auto ks_part = [&]() {
-        f32x4 ak[4];
-#pragma unroll
-        for (int tt = 0; tt < 4; tt++) ak[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kc = 0; kc < 4; kc++) {
-          bf16x8 kr[4];
-#pragma unroll
-          for (int tt = 0; tt < 4; tt++) kr[tt] = ld8(Kc, ((16 * tt + c16) * P136 + 32 * kc + 8 * q4) * 2);
-#pragma unroll
-          for (int tt = 0; tt < 4; tt++) ak[tt] = mfma(kr[tt], sh[kc], ak[tt]);
-#pragma unroll
-          for (int tt = 0; tt < 4; tt++) ak[tt] = mfma(kr[tt], sl[kc], ak[tt]);
-        }
-#pragma unroll
-        for (int tt = 0; tt < 4; tt++) {
-          const int ta = 16 * tt + 4 * q4;
-          const float4 be = *(const float4 *)(sm + SM_BETA * 64 + ta), gk = *(const float4 *)(sm + SM_GK * 64 + ta);
-          const float be4[4] = {be.x, be.y, be.z, be.w}, gk4[4] = {gk.x, gk.y, gk.z, gk.w};
-          const tr4_t vr = col4(Vc, ta, jw, c16);  // v of tokens ta .. ta + 3, column jw + c16
-          const float v4[4] = {bf2f((uint16_t)vr[0]), bf2f((uint16_t)vr[1]), bf2f((uint16_t)vr[2]),
-                               bf2f((uint16_t)vr[3])};
-#pragma unroll
-          for (int r = 0; r < 4; r++) R[tt][r] = be4[r] * (v4[r] - gk4[r] * ak[tt][r]);
-        }
-      };
+      auto ks_part = [&]() { ks_of(sh, sl, R, true); };
       auto qs_part = [&]() {
         f32x4 aq[4];
 #pragma unroll
@@ -3967,7 +4026,19 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
       // tiles below the diagonal, two of them split into their A and P
       // halves, so that each SIMD (waves w and w + 4) holds two and a half
       // tile pairs and one diagonal solve
-      switch (__builtin_amdgcn_readfirstlane(w)) {
+      // (SUMMARY: A tiles only, the six below the diagonal on waves 4-7)
+      if constexpr (SUMMARY) {
+        switch (__builtin_amdgcn_readfirstlane(w)) {
+          case 0: ap_tile(0, 0, true, false); ks_part(); diag_solve(0); break;
+          case 1: ap_tile(1, 1, true, false); ks_part(); diag_solve(1); break;
+          case 2: ap_tile(2, 2, true, false); ks_part(); diag_solve(2); break;
+          case 3: ap_tile(3, 3, true, false); ks_part(); diag_solve(3); break;
+          case 4: ap_tile(3, 0, true, false); ks_part(); ap_tile(3, 1, true, false); break;
+          case 5: ap_tile(3, 2, true, false); ks_part(); ap_tile(1, 0, true, false); break;
+          case 6: ap_tile(2, 0, true, false); ks_part(); break;
+          default: ap_tile(2, 1, true, false); ks_part(); break;
+        }
+      } else switch (__builtin_amdgcn_readfirstlane(w)) {
         case 0: ap_tile(0, 0); ks_part(); diag_solve(0); qs_part(); break;
         case 1: ap_tile(1, 1); ks_part(); diag_solve(1); qs_part(); break;
         case 2: ap_tile(2, 2); ks_part(); diag_solve(2); qs_part(); break;
@@ -3989,9 +4060,10 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
     // the permuted slot order.  Delta' = diag(nk Gamma_C / Gamma) Delta.
     f32x4 dp[4];
     bf16x8 ph01, pl01, ph23, pl23;  // [D_0; D_1] and [D_2; D_3] (hi, lo), permuted slots
-    {
+    auto delta_solve = [&](const f32x4 (&R)[4]) {
       const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
       bf16x4 xh[4], xl[4];
+      f32x4 c0, c1;
       // acc + M[16 i .. 16 i + 15][16 k .. 16 k + 15] x (hi/lo pairs hi*hi + hi*lo + lo*hi)
       auto mone = [&](int i, int k, bf16x4 bh, bf16x4 bl, f32x4 acc) {
         const int o = ((16 * i + c16) * P72 + pcol(16 * k + 4 * q4)) * 2;
@@ -4004,9 +4076,9 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
       auto mpair = [&](int i, f32x4 acc) {
         const int o = ((16 * i + c16) * P72 + 8 * q4) * 2;
         const bf16x8 mh = ld8(Tb, o), ml = ld8(Tb, PC * P72 * 2 + o);
-        acc = mfma(mh, ph01, acc);
-        acc = mfma(mh, pl01, acc);
-        return mfma(ml, ph01, acc);
+        c0 = mfma(mh, ph01, acc);
+        c1 = mfma(mh, pl01, c0);
+        return mfma(ml, ph01, c1);
       };
 #pragma unroll
       for (int i = 0; i < 4; i++) {
@@ -4016,7 +4088,12 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
         if (i == 3) acc = mone(3, 2, xh[2], xl[2], acc);
         bf16x4 ah, al;
         split4x(acc, ah, al);
-        const f32x4 d = mone(i, i, ah, al, zero);
+        f32x4 d = mone(i, i, ah, al, zero);
+        // the chain's accumulator inputs stay allocated until its result: a
+        // register of theirs rewritten a few instructions after the product
+        // that reads it (nothing else held it) gave wrong rows of D_3 in the
+        // summary kernel, differently from run to run
+        if (i >= 2) asm volatile("" : "+v"(d) : "v"(c0), "v"(c1), "v"(R[i]));
         split4x(d, xh[i], xl[i]);
         if (i == 1) {
           ph01 = cat8(xh[0], xh[1]);
@@ -4032,13 +4109,14 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
         dp[i][2] = d[2] * kd.z;
         dp[i][3] = d[3] * kd.w;
       }
-    }
+    };
+    delta_solve(R);
     // ---- O^T = diag(nq Gamma) (S0^T Q^T) + Delta^T P^T: rows j of this wave,
     // column t; a split pair [D_2kc; D_2kc+1] is the A operand of its
     // transpose as it is, and token pairs past the tile are causal zeros
     // (the six tile pairs' loads first, then their products interleaved
     // across the four independent token tiles)
-    {
+    if constexpr (!SUMMARY) {
       bf16x8 ph[6], pl[6];
 #pragma unroll
       for (int e = 0; e < 6; e++) {
@@ -4074,7 +4152,7 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
     }
     // ---- S <- Gamma_C S0 + K^T Delta' (rows d, this wave's columns; tokens
     // in the permuted slot order, two 4-token runs of the k column each)
-    {
+    auto state_update = [&](f32x4 (&S)[8]) {
       bf16x8 eh[2], el[2];
       split8(dp[0], dp[1], eh[0], el[0]);
       split8(dp[2], dp[3], eh[1], el[1]);
@@ -4100,6 +4178,20 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
           for (int dt = d4; dt < d4 + 4; dt++) S[dt] = mfma(a[dt - d4][kc], el[kc], S[dt]);
         }
       }
+    };
+    state_update(S);
+    if constexpr (SUMMARY) {
+      if (trans) {
+        // M's columns after E's, not beside them: both sets of operands at
+        // once exceed the 256 registers of two waves per SIMD
+        __builtin_amdgcn_sched_barrier(0);
+        bf16x8 sh[4], sl[4];
+#pragma unroll
+        for (int kc = 0; kc < 4; kc++) split8(M[2 * kc], M[2 * kc + 1], sh[kc], sl[kc]);
+        ks_of(sh, sl, R, false);
+        delta_solve(R);
+        state_update(M);
+      }
     }
     lds_barrier();  // the next chunk's staging overwrites the shared tiles
     c0 = c_next;
@@ -4115,6 +4207,90 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
           for (int r = 0; r < 4; r++) dst[(int64_t)(16 * dt + 4 * q4 + r) * PV] = S[dt][r];
       }
     }
+  }
+  if constexpr (SUMMARY) {
+    const int64_t at = ((int64_t)sg.slot * H + h) * PKD * PV + jw + c16;
+#pragma unroll
+    for (int dt = 0; dt < 8; dt++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        D.seg_state[at + (int64_t)(16 * dt + 4 * q4 + r) * PV] = S[dt][r];
+        if (trans) D.seg_trans[at + (int64_t)(16 * dt + 4 * q4 + r) * PV] = M[dt][r];
+      }
+  }
+}
+
+// Start states of a sequence's segments from the segments' summaries: on
+// entry seg_state[s] is E_s (s = 0: the state after segment 0), on exit the
+// state after segment s, S_{s+1} = M_s S_s + E_s for s = 1 .. the last but
+// one.  State columns are independent: a workgroup takes 16 columns of one
+// (sequence, head), wave w the rows 16 w .. 16 w + 15, with the 128 x 16 state
+// handed from wave to wave through LDS as hi/lo bf16 (products hi*hi + hi*lo
+// + lo*hi, as in the recurrence).  Bound by the loads of M, 64 KB a step:
+// those of the next two segments are in flight behind each step's products,
+// and the eight workgroups that read one M sit on one XCD (grid x is
+// sequences x heads, dealt to the XCDs in turn).
+constexpr int CB_PITCH = 136;  // elements of a column in the LDS copy of the state
+__global__ __launch_bounds__(NT) void segment_combine_kernel(PrefillDev D) {
+#pragma clang fp contract(off)
+  __shared__ __align__(16) uint16_t st[2][2][16 * CB_PITCH];  // [buffer][hi, lo][column][row]
+  const int H = D.H, h = blockIdx.x % H, b = blockIdx.x / H, jw = 16 * blockIdx.y;
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, q4 = l >> 4, c16 = l & 15;
+  const Segment first = segment_of(D, b, 0);
+  const int len = __builtin_amdgcn_readfirstlane(D.cu[b + 1]) - first.t0;
+  const int n = len > 0 ? (len - 1) / D.seg : 0;  // summaries 0 .. n - 1: segments but the last
+  if (n < 2) return;
+  const int64_t step = (int64_t)H * PKD * PV;
+  float *state = D.seg_state + ((int64_t)first.slot * H + h) * PKD * PV + jw + (16 * w + 4 * q4) * PV + c16;
+  const float *trans = D.seg_trans + ((int64_t)first.slot * H + h) * PKD * PV + (16 * w + c16) * PV + 4 * q4;
+  f32x4 m[2][4][2];  // of two segments: row 16 w + c16, columns 32 kb + 16 i + 4 q4 .. + 3
+  f32x4 e[2], x;     // rows 16 w + 4 q4 + r of column jw + c16
+  auto load = [&](int s, f32x4 (&mm)[4][2], f32x4 &ee) {
+    const int64_t at = step * (s < n ? s : n - 1);
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) mm[kb][i] = *(const f32x4 *)(trans + at + 32 * kb + 16 * i);
+#pragma unroll
+    for (int r = 0; r < 4; r++) ee[r] = state[at + r * PV];
+  };
+#pragma unroll
+  for (int r = 0; r < 4; r++) x[r] = state[r * PV];
+  load(1, m[0], e[0]);
+  load(2, m[1], e[1]);
+  auto one = [&](int s, f32x4 (&mm)[4][2], f32x4 &ee, int buf) {
+    uint2 hi, lo;
+    split2(x[0], x[1], hi.x, lo.x);
+    split2(x[2], x[3], hi.y, lo.y);
+    const int put = c16 * CB_PITCH + pcol(16 * w + 4 * q4);  // rows in split8's slot order
+    *(uint2 *)(st[buf][0] + put) = hi;
+    *(uint2 *)(st[buf][1] + put) = lo;
+    bf16x8 mh[4], ml[4];
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++) split8(mm[kb][0], mm[kb][1], mh[kb], ml[kb]);
+    x = ee;
+    load(s + 2, mm, ee);
+    // one barrier a segment: the other buffer's readers are past theirs
+    lds_barrier();
+    f32x4 y = {0.f, 0.f, 0.f, 0.f};  // two chains: blocks 0, 1 and 2, 3
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++) {
+      const int at = (c16 * CB_PITCH + 32 * kb + 8 * q4) * 2;
+      const bf16x8 sh = ld8((const uint8_t *)st[buf][0], at), sl = ld8((const uint8_t *)st[buf][1], at);
+      f32x4 &acc = kb < 2 ? x : y;
+      acc = mfma(mh[kb], sh, acc);
+      acc = mfma(mh[kb], sl, acc);
+      acc = mfma(ml[kb], sh, acc);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      x[r] = x[r] + y[r];
+      state[step * s + r * PV] = x[r];
+    }
+  };
+  for (int s = 1; s < n; s += 2) {
+    one(s, m[0], e[0], 0);
+    if (s + 1 < n) one(s + 1, m[1], e[1], 1);
   }
 }
 
@@ -5811,7 +5987,59 @@ int sq_create_cu_stream(int32_t device, int32_t cus, void **stream, int32_t *act
   return 0;
 }
 
+int sq_prefill_plan(const sq_pool *pool, const int32_t *cu, int64_t batch, int32_t cus, sq_prefill_segments *out) {
+  if (!pool || !cu || !out || batch < 0) return fail(SQ_EINVAL, "prefill plan: null argument or negative batch");
+  *out = sq_prefill_segments{0, 0, 0, nullptr};
+  if (pool->kda) return 0;
+  if (cus <= 0) {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      return check_launch("prefill plan: device query");
+    cus = n;
+  }
+  const int64_t H = pool->heads;
+  if (batch == 0 || H < 1 || batch * H > cus) return 0;
+  // Time of a call whose workgroups all fit the device at once (one per
+  // compute unit), measured in microseconds: whole sequences take 6.1 a
+  // 64-token chunk (32 workgroups), one after the other; cut into P segments,
+  // every segment's summary and full pass take 7.9 + 7.7 a chunk (256
+  // workgroups) over longest / P tokens, and the combine 2.5 a segment.
+  // (B = 1, T = 8192, 32 heads: 785 us whole, 127 + 125 + 20 us in 8
+  // segments.)  A split that saves less than 15% is not taken.
+  const double whole_chunk = 6.1, split_chunk = 15.6, step = 2.5, extra = 8.0;
+  const int64_t C = pf::PC;
+  int64_t longest = 0;
+  for (int64_t b = 0; b < batch; b++) longest = cu[b + 1] - cu[b] > longest ? cu[b + 1] - cu[b] : longest;
+  double best = .85 * whole_chunk * (double)((longest + C - 1) / C);
+  for (int64_t P = 2; P * H <= cus && P * C < longest + C; P++) {
+    const int64_t L = ((longest + P - 1) / P + C - 1) / C * C;
+    int64_t whole = 0, summaries = 0;
+    for (int64_t b = 0; b < batch; b++) {
+      const int64_t len = cu[b + 1] - cu[b], n = len > 0 ? (len + L - 1) / L : 0;
+      whole += n;
+      summaries += n > 1 ? n - 1 : 0;
+    }
+    if (whole * H > cus || summaries * H > cus) break;
+    const double t = split_chunk * (double)(L / C) + step * (double)P + extra;
+    if (t < best) {
+      best = t;
+      out->tokens = (int32_t)L;
+      out->count = (int32_t)((longest + L - 1) / L);
+    }
+  }
+  if (out->tokens) {
+    const int64_t slots = cu[batch] / out->tokens + batch;
+    out->workspace_bytes = 2 * slots * H * 128 * 128 * (int64_t)sizeof(float);
+  }
+  return 0;
+}
+
 int sq_prefill(const sq_pool *pool, const sq_prefill_args *a, void *stream) {
+  return sq_prefill_split(pool, a, nullptr, stream);
+}
+
+int sq_prefill_split(const sq_pool *pool, const sq_prefill_args *a, const sq_prefill_segments *sg, void *stream) {
   int rc = validate_pool(pool);
   if (rc) return rc;
   if (!a) return fail(SQ_EINVAL, "prefill: null arguments");
@@ -5842,6 +6070,16 @@ int sq_prefill(const sq_pool *pool, const sq_prefill_args *a, void *stream) {
   if (a->q_stride < 0 || a->k_stride < 0 || a->v_stride < 0 || a->q_stride >= (1 << 23) || a->k_stride >= (1 << 23) ||
       a->v_stride >= (1 << 23))
     return fail(SQ_EINVAL, "prefill: q, k, v row strides must be below 2^23 elements");
+  const bool split = sg && sg->tokens > 0;
+  if (split) {
+    const int64_t state = (int64_t)pool->heads * 128 * 128 * (int64_t)sizeof(float);
+    if (pool->kda || sg->tokens % pf::PC || sg->count < 2 || sg->count > 16384 || a->batch > 65535 ||
+        pool->heads > 65535)
+      return fail(SQ_EINVAL, "prefill: segments must be whole chunks, two or more a sequence");
+    if (!sg->workspace || ((uintptr_t)sg->workspace & 15) || sg->workspace_bytes < 2 * state * a->batch ||
+        sg->workspace_bytes % (2 * state))
+      return fail(SQ_EINVAL, "prefill: segments need the planned workspace, 16-byte aligned");
+  }
   hipStream_t st = (hipStream_t)stream;
   const int H = pool->heads;
   const int64_t dense = a->batch * (int64_t)H * 128 * 128;
@@ -5896,6 +6134,9 @@ int sq_prefill(const sq_pool *pool, const sq_prefill_args *a, void *stream) {
   D.pi.slots = a->init_slots;
   D.pi.slots_dtype = a->slots_dtype;
   D.pi.ng = pool->group >= 32 ? 128 / pool->group : 1;
+  D.seg = split ? sg->tokens : 0;
+  D.seg_state = split ? (float *)sg->workspace : nullptr;
+  D.seg_trans = split ? D.seg_state + sg->workspace_bytes / (2 * sizeof(float)) : nullptr;
   if (pool->kda) {
     hipError_t e = hipFuncSetAttribute((const void *)kc::kda_chunk_kernel,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, kc::LDS_BYTES);
@@ -5905,12 +6146,24 @@ int sq_prefill(const sq_pool *pool, const sq_prefill_args *a, void *stream) {
     hipLaunchKernelGGL(kc::kda_chunk_kernel, dim3((unsigned)(a->batch * H)), dim3(kc::NT), kc::LDS_BYTES, st, D);
     rc = check_launch("kda_chunk_kernel");
   } else {
-    hipError_t e = hipFuncSetAttribute((const void *)pf::prefill_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       pf::LDS_BYTES);
+    hipError_t e = hipFuncSetAttribute((const void *)pf::prefill_kernel<false>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, pf::LDS_BYTES);
+    if (e == hipSuccess && split)
+      e = hipFuncSetAttribute((const void *)pf::prefill_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              pf::LDS_BYTES);
     if (e != hipSuccess) return fail((int)e, "prefill: cannot raise the kernel's LDS limit");
     if (a->events && (e = hipEventRecord((hipEvent_t)a->events[0], st)) != hipSuccess)
       return fail((int)e, "prefill: hipEventRecord failed");
-    hipLaunchKernelGGL(pf::prefill_kernel, dim3((unsigned)(a->batch * H)), dim3(pf::NT), pf::LDS_BYTES, st, D);
+    const unsigned tiles = (unsigned)(a->batch * H), count = split ? (unsigned)sg->count : 1u;
+    if (split) {
+      hipLaunchKernelGGL(pf::prefill_kernel<true>, dim3(tiles, count - 1), dim3(pf::NT), pf::LDS_BYTES, st, D);
+      if ((rc = check_launch("prefill_kernel (segment summaries)"))) return rc;
+      if (count > 2) {
+        hipLaunchKernelGGL(pf::segment_combine_kernel, dim3(tiles, 8), dim3(pf::NT), 0, st, D);
+        if ((rc = check_launch("segment_combine_kernel"))) return rc;
+      }
+    }
+    hipLaunchKernelGGL(pf::prefill_kernel<false>, dim3(tiles, count), dim3(pf::NT), pf::LDS_BYTES, st, D);
     rc = check_launch("prefill_kernel");
   }
   if (rc) return rc;

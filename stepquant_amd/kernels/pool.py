@@ -374,19 +374,16 @@ class PackedStatePool:
         cu_host = None
         if isinstance(cu_seqlens, torch.Tensor) and cu_seqlens.device.type != "cpu":
             cu = cu_seqlens.to(dev, torch.int32).reshape(-1).contiguous()
-            total = 0
-            if cu.numel() > 1:
-                # one wait for the stream: the row count and the offsets' validity
-                first, total, drops = torch.stack([cu[0], cu[-1], (cu[1:] < cu[:-1]).sum().to(torch.int32)]).tolist()
-                _check_offsets(first, drops)
+            offsets = cu.cpu()  # one wait for the stream: the row count, the offsets' validity, the lengths
         else:
             # offsets known on the host: checked here, copied without a wait
-            cu_host = torch.as_tensor(cu_seqlens).to(torch.int32).reshape(-1)
-            total = int(cu_host[-1]) if cu_host.numel() > 1 else 0
-            if cu_host.numel() > 1:
-                _check_offsets(int(cu_host[0]), int((cu_host[1:] < cu_host[:-1]).sum()))
+            cu_host = offsets = torch.as_tensor(cu_seqlens).to(torch.int32).reshape(-1).contiguous()
             cu = None  # copied below, with the checkpoints when they are host tensors too
-        batch = (cu if cu_host is None else cu_host).numel() - 1
+        total = 0
+        if offsets.numel() > 1:
+            total = int(offsets[-1])
+            _check_offsets(int(offsets[0]), int((offsets[1:] < offsets[:-1]).sum()))
+        batch = offsets.numel() - 1
         if batch < 0:
             raise ValueError("cu_seqlens needs at least one entry")
         slots_t = _indices(slots, dev)
@@ -497,7 +494,11 @@ class PackedStatePool:
             ev = (ctypes.c_void_p * 2)(*handles)
             args.events = ctypes.cast(ev, ctypes.c_void_p)
         if batch:
-            N.check(N.lib().sq_prefill(self._desc, args, N.stream_handle()), "prefill")
+            segments = N.prefill_plan(self._desc, offsets)
+            if segments.tokens:
+                workspace = torch.empty(segments.workspace_bytes, device=dev, dtype=torch.uint8)
+                segments.workspace = workspace.data_ptr()
+            N.check(N.lib().sq_prefill_split(self._desc, args, segments, N.stream_handle()), "prefill")
         if keep:
             self.last_prefill = (q2, k2, v2, g2, b2, al, db, cu, ck, init, ck_slots, init_state, ck_state)
         return out

@@ -1,0 +1,93 @@
+"""Prefill with sequences cut into segments (sq_prefill_plan / sq_prefill_split, MI355X).
+
+Gates that forget slowly (down to 1e-3 a token) carry the state across
+segments, so an error in a segment's transition or start state shows.  Bars
+as for whole sequences: states rtol 1e-3 / atol 1e-4 of the float64
+recurrence, outputs rtol 2^-8 / atol 1e-4; the transitions add products of
+the same hi/lo operands (~2^-17 relative), one per segment.
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from tests.helpers import check_prefill, check_states, dev, device_plan, make_plan
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(arch, lens, ck, tokens, monkeypatch, storage="packed", cu_on_device=False):
+    from stepquant_amd import _native as N
+    from stepquant_amd.kernels.pool import PackedStatePool
+    H, HK, K, V = 4, 4 if arch == "kda" else 2, 128, 128
+    B, NC = np.shape(ck)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    T = int(cu[-1])
+    rng = np.random.default_rng(3)
+    bits = np.repeat(np.array([6, 8, 4, 6])[:, None], K, 1) if arch == "gdn" else rng.choice([4, 6, 8, 16], (H, K))
+    stream = torch.cuda.Stream() if storage == "byte" else None
+    pool = PackedStatePool(device_plan(make_plan(arch, bits, seed=3)), B * (NC + 1) + 1, V, storage=storage,
+                           writeback_stream=stream)
+    g = torch.Generator().manual_seed(11)
+    q, k = (torch.randn(T, HK, K, generator=g).to(torch.bfloat16) for _ in range(2))
+    v = torch.randn(T, H, V, generator=g).to(torch.bfloat16)
+    shape = (T, H, K) if arch == "kda" else (T, H)
+    rate = torch.tensor([1e-3, 5e-3, 5e-2, .5]).reshape(1, H, *([1] * (len(shape) - 2)))
+    gate = -rate * torch.rand(shape, generator=g) * 2
+    beta = torch.rand(T, H, generator=g)
+    init = torch.arange(B)  # slot 0: the first sequence starts from zero
+    pool.encode((torch.randn(B, H, K, V, generator=g) * .5).to(dev()), init.to(dev()))
+    pool.wait()
+    torch.cuda.synchronize()
+    lay = O.layout(make_plan(arch, bits, seed=3), V, storage)
+    S0 = O.decode_page(pool.data.cpu().numpy(), init.numpy(), make_plan(arch, bits, seed=3), lay, V,
+                       storage).astype(np.float64)
+    seen = []
+    if tokens:
+        def plan(desc, offsets, cus=0):
+            slots = int(offsets[-1]) // tokens + B
+            seen.append(N.PrefillSegments(tokens, -(-max(lens) // tokens), 2 * slots * H * K * V * 4, None))
+            return seen[-1]
+    else:
+        whole = N.prefill_plan
+
+        def plan(desc, offsets, cus=0):
+            seen.append(whole(desc, offsets, cus))
+            return seen[-1]
+    monkeypatch.setattr(N, "prefill_plan", plan)
+    pool.keep_prefill_states = True
+    offsets = torch.from_numpy(cu)
+    out = pool.extend(q.to(dev()), k.to(dev()), v.to(dev()), gate.to(dev()), beta.to(dev()), init,
+                      offsets.to(dev()) if cu_on_device else offsets, checkpoints=torch.tensor(ck),
+                      checkpoint_slots=torch.arange(B, B + B * NC).reshape(B, NC), init_slots=init, normalize=True,
+                      scale=K ** -.5)
+    torch.cuda.synchronize()
+    assert seen[0].tokens and seen[0].count >= 2
+    ref_out, ref_states, _ = O.prefill(q.float().numpy(), k.float().numpy(), v.float().numpy(), gate.numpy(),
+                                       beta.numpy(), S0, cu, ck, normalize=True, scale=K ** -.5)
+    states = pool.last_prefill[-1].cpu().numpy().reshape(B, NC, H, K, V)
+    check_prefill(out, ref_out, f"{arch} {storage} tokens={tokens}")
+    for b in range(B):
+        for c in range(NC):
+            if 0 < ck[b][c] <= lens[b]:
+                check_states(states[b, c], ref_states[b, c], f"state b={b} c={c}")
+
+
+# lengths: below, at and past a segment, empty, one token, many segments;
+# checkpoints inside, at and just past a segment's end
+LENS = [640, 0, 128, 129, 1, 333]
+MARKS = [[128, 640], [0, 0], [64, 128], [128, 129], [1, 0], [130, 333]]
+
+
+@pytest.mark.parametrize("arch,tokens", [("gdn", 64), ("gdn", 128), ("gdn", 320)])
+def test_segments_against_the_recurrence(arch, tokens, monkeypatch):
+    print(f"case {arch} tokens={tokens}", flush=True)
+    _case(arch, LENS, MARKS, tokens, monkeypatch)
+
+
+@pytest.mark.parametrize("arch,storage", [("gdn", "packed"), ("gdn", "byte")])
+def test_planned_segments_against_the_recurrence(arch, storage, monkeypatch):
+    """The plan's own choice, offsets on the device, byte pages (dense
+    initial states) and packed ones."""
+    print(f"case {arch} {storage} planned", flush=True)
+    _case(arch, [1500, 70], [[700, 1500], [64, 70]], 0, monkeypatch, storage, cu_on_device=True)
