@@ -4533,15 +4533,22 @@ __device__ __forceinline__ void kda_init_from_page(const pf::PageInit &pi, int b
     }
 }
 
+// One workgroup per (sequence, head), or with D.seg per (sequence segment,
+// head), blockIdx.y the segment; SUMMARY: the segment's E and M instead of
+// outputs and checkpoints, as pf::prefill_kernel (the per-channel decay
+// scales rows, so state columns pass through the recurrence alone here too).
+template <bool SUMMARY>
 __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
 #pragma clang fp contract(off)
   extern __shared__ __align__(16) uint8_t smem[];
   const int H = D.H;
   const int h = blockIdx.x % H, b = blockIdx.x / H;
   const int hk = h / (H / D.HK);
-  const int t0 = __builtin_amdgcn_readfirstlane(D.cu[b]);
-  const int len = __builtin_amdgcn_readfirstlane(D.cu[b + 1]) - t0;
-  if (len <= 0) return;  // whole workgroup
+  const int seg_i = blockIdx.y;
+  const bool trans = SUMMARY && seg_i > 0;  // M wanted
+  const pf::Segment sg = pf::segment_of(D, b, seg_i);
+  const int t0 = sg.t0, len = sg.len;
+  if (len <= 0 || (SUMMARY && sg.last)) return;  // whole workgroup
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, q4 = l >> 4, c16 = l & 15;
   const int jw = 16 * w;
   uint8_t *VR = smem + OFF_VR;
@@ -4561,18 +4568,31 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
   pf::lds_barrier();
 
   // ---- state S[d][j] of this wave's columns: tile dt holds rows d = 16 dt + 4 q4 + r, column jw + c16
-  f32x4 S[8];
-  if (D.page_init) {
+  f32x4 S[8], MS[SUMMARY ? 8 : 1];  // MS: the same columns of the segment's M
+  if constexpr (SUMMARY) {
+#pragma unroll
+    for (int dt = 0; dt < 8; dt++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        MS[dt][r] = 16 * dt + 4 * q4 + r == jw + c16 ? 1.0f : 0.0f;
+        S[dt][r] = 0.0f;
+      }
+  }
+  if (SUMMARY && seg_i > 0) {
+    // E from zero
+  } else if (D.page_init && seg_i == 0) {
     kda_init_from_page(D.pi, b, h, H, smem, tid, S);
     __syncthreads();  // the staged page is read before the first chunk's tiles overwrite it
   } else {
-    const float *src = D.init + ((int64_t)b * H + h) * KV * KV + jw + c16;
+    // the sequence's dense initial state, or the segment's start state
+    const float *src = (seg_i == 0 ? D.init + ((int64_t)b * H + h) * KV * KV
+                                   : D.seg_state + ((int64_t)(sg.slot - 1) * H + h) * KV * KV) + jw + c16;
 #pragma unroll
     for (int dt = 0; dt < 8; dt++)
 #pragma unroll
       for (int r = 0; r < 4; r++) S[dt][r] = src[(int64_t)(16 * dt + 4 * q4 + r) * KV];
   }
-  const int ckv = l < D.NC ? D.ckpt[(int64_t)b * D.NC + l] : 0x7fffffff;
+  const int ckv = !SUMMARY && l < D.NC ? D.ckpt[(int64_t)b * D.NC + l] - sg.start : 0x7fffffff;
   auto segment = [&](int c) {  // tokens of the chunk at c: up to the next checkpoint, the end, or C
     const uint64_t m = __ballot(ckv > c && ckv <= len);
     const int stop = m ? __builtin_amdgcn_readlane(ckv, __builtin_ctzll(m)) : len;
@@ -4586,10 +4606,12 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
   const uint8_t *qg = (const uint8_t *)D.q, *kg = (const uint8_t *)D.k, *vg = (const uint8_t *)D.v;
   auto fetch = [&](Fetch &F, int c) {
     F.n = c < len ? segment(c) : 0;
+    const int tid = SUMMARY ? fast::opaque(threadIdx.x) : (int)threadIdx.x, l = tid & 63;
+    const int tt = tid >> 4, c8 = (tid & 15) * 8, gc = tid >> 2, gq = tid & 3;
     const int last = len - 1;
     const int64_t row = (int64_t)t0 + (c + tt < len ? c + tt : last);
     F.k = *(const uint4 *)(kg + (row * D.k_stride + (int64_t)hk * KV + c8) * 2);
-    F.q = *(const uint4 *)(qg + (row * D.q_stride + (int64_t)hk * KV + c8) * 2);
+    if (!SUMMARY) F.q = *(const uint4 *)(qg + (row * D.q_stride + (int64_t)hk * KV + c8) * 2);
     F.v = *(const uint4 *)(vg + (row * D.v_stride + (int64_t)h * KV + c8) * 2);
 #pragma unroll
     for (int i = 0; i < 8; i++) {
@@ -4605,25 +4627,28 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
   // rows, raw k and q rows, norms, beta; cumulative decays per channel
   auto stage_chunk = [&](int pa) {
     const int n = F.n;
+    const int tid = SUMMARY ? fast::opaque(threadIdx.x) : (int)threadIdx.x, l = tid & 63;
+    const int tt = tid >> 4, c8 = (tid & 15) * 8, gc = tid >> 2, gq = tid & 3;
     float kf[8], qf[8];
     bf8(F.k, kf);
-    bf8(F.q, qf);
+    if (!SUMMARY) bf8(F.q, qf);
     const bool live = tt < n;
     const uint32_t mk = live ? 0xffffffffu : 0u;  // tokens past the chunk's: zero rows
     *(uint4 *)(KB + (tt * RP + c8) * 2) = make_uint4(F.k.x & mk, F.k.y & mk, F.k.z & mk, F.k.w & mk);
-    *(uint4 *)(QB + (tt * RP + c8) * 2) = make_uint4(F.q.x & mk, F.q.y & mk, F.q.z & mk, F.q.w & mk);
+    if (!SUMMARY) *(uint4 *)(QB + (tt * RP + c8) * 2) = make_uint4(F.q.x & mk, F.q.y & mk, F.q.z & mk, F.q.w & mk);
     *(uint4 *)(VR + (tt * RP + c8) * 2) = make_uint4(F.v.x & mk, F.v.y & mk, F.v.z & mk, F.v.w & mk);
     float sk = 0.f, sq = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; e++) {
       sk = fmaf(kf[e], kf[e], sk);
-      sq = fmaf(qf[e], qf[e], sq);
+      if (!SUMMARY) sq = fmaf(qf[e], qf[e], sq);
     }
     sk = pf::row16_sum(sk);
-    sq = pf::row16_sum(sq);
+    if (!SUMMARY) sq = pf::row16_sum(sq);
     if ((tid & 15) == 0) {
       sm[SM_NK * C + tt] = live && D.normalize ? __builtin_amdgcn_rsqf(sk + 1e-6f) : (live ? 1.0f : 0.0f);
-      sm[SM_NQ * C + tt] = live ? (D.normalize ? __builtin_amdgcn_rsqf(sq + 1e-6f) : 1.0f) * D.scale : 0.0f;
+      if (!SUMMARY)
+        sm[SM_NQ * C + tt] = live ? (D.normalize ? __builtin_amdgcn_rsqf(sq + 1e-6f) : 1.0f) * D.scale : 0.0f;
     }
     if (w == 0 && l < C) {
       float bt = F.beta;
@@ -4665,12 +4690,16 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
   pf::lds_barrier();
   for (int c0 = 0; c0 < len; par ^= 1) {
     const int c_next = c0 + n;
+    // SUMMARY: lane indices re-derived each chunk (see pf::prefill_kernel), so
+    // that LDS addresses are not held in registers across the loop
+    const int tid = SUMMARY ? fast::opaque(threadIdx.x) : (int)threadIdx.x, l = tid & 63, q4 = l >> 4, c16 = l & 15;
+    const int tt = tid >> 4, c8 = (tid & 15) * 8;
     const bool pairwise = sm[SM_FLAG * C + par] != 0.0f;  // workgroup-uniform
     // ---- operands of token tt, channels c8 .. c8 + 7: nk k e^G and nq q e^G
     // (hi/lo, pcol order), nk k e^{G_C - G} (hi/lo), e^{G_C}; for the MFMA path
     // k e^{G - G_C} and q e^{G - G_C} (hi/lo) in place of the raw rows
     {
-      const float nk = sm[SM_NK * C + tt], nq = sm[SM_NQ * C + tt];
+      const float nk = sm[SM_NK * C + tt], nq = SUMMARY ? 0.0f : sm[SM_NQ * C + tt];
       float g8[8], gc8[8];
       {
         const float4 a0 = *(const float4 *)(G + tt * GP + c8), a1 = *(const float4 *)(G + tt * GP + c8 + 4);
@@ -4685,29 +4714,31 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
       }
       float kf[8], qf[8];
       bf8(*(const uint4 *)(KB + (tt * RP + c8) * 2), kf);
-      bf8(*(const uint4 *)(QB + (tt * RP + c8) * 2), qf);
+      if (!SUMMARY) bf8(*(const uint4 *)(QB + (tt * RP + c8) * 2), qf);
       float kgv[8], qgv[8], kdv[8];
 #pragma unroll
       for (int e = 0; e < 8; e++) {
         const float eg = __builtin_amdgcn_exp2f(g8[e]);
         kgv[e] = (nk * kf[e]) * eg;
-        qgv[e] = (nq * qf[e]) * eg;
+        if (!SUMMARY) qgv[e] = (nq * qf[e]) * eg;
         kdv[e] = (nk * kf[e]) * __builtin_amdgcn_exp2f(gc8[e] - g8[e]);
       }
       {
         // channels c8 .. c8 + 3 and c8 + 4 .. c8 + 7 at their permuted places
         uint4 kh8, kl8, qh8, ql8;
         split8v(kgv, kh8, kl8);
-        split8v(qgv, qh8, ql8);
         const int p0 = pf::pcol(c8), p1 = pf::pcol(c8 + 4);
         *(uint2 *)(KG + (tt * RP + p0) * 2) = make_uint2(kh8.x, kh8.y);
         *(uint2 *)(KG + (tt * RP + p1) * 2) = make_uint2(kh8.z, kh8.w);
         *(uint2 *)(KG + KB_LO + (tt * RP + p0) * 2) = make_uint2(kl8.x, kl8.y);
         *(uint2 *)(KG + KB_LO + (tt * RP + p1) * 2) = make_uint2(kl8.z, kl8.w);
-        *(uint2 *)(QG + (tt * RP + p0) * 2) = make_uint2(qh8.x, qh8.y);
-        *(uint2 *)(QG + (tt * RP + p1) * 2) = make_uint2(qh8.z, qh8.w);
-        *(uint2 *)(QG + KB_LO + (tt * RP + p0) * 2) = make_uint2(ql8.x, ql8.y);
-        *(uint2 *)(QG + KB_LO + (tt * RP + p1) * 2) = make_uint2(ql8.z, ql8.w);
+        if constexpr (!SUMMARY) {
+          split8v(qgv, qh8, ql8);
+          *(uint2 *)(QG + (tt * RP + p0) * 2) = make_uint2(qh8.x, qh8.y);
+          *(uint2 *)(QG + (tt * RP + p1) * 2) = make_uint2(qh8.z, qh8.w);
+          *(uint2 *)(QG + KB_LO + (tt * RP + p0) * 2) = make_uint2(ql8.x, ql8.y);
+          *(uint2 *)(QG + KB_LO + (tt * RP + p1) * 2) = make_uint2(ql8.z, ql8.w);
+        }
       }
       uint4 h4, l4;
       split8v(kdv, h4, l4);
@@ -4719,14 +4750,16 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
         for (int e = 0; e < 8; e++) {
           const float eb = __builtin_amdgcn_exp2f(g8[e] - gc8[e]);
           kbv[e] = kf[e] * eb;
-          qbv[e] = qf[e] * eb;
+          if (!SUMMARY) qbv[e] = qf[e] * eb;
         }
         split8v(kbv, h4, l4);
         *(uint4 *)(KB + (tt * RP + c8) * 2) = h4;  // over this thread's own raw entries
         *(uint4 *)(KB + KB_LO + (tt * RP + c8) * 2) = l4;
-        split8v(qbv, h4, l4);
-        *(uint4 *)(QB + (tt * RP + c8) * 2) = h4;
-        *(uint4 *)(QB + KB_LO + (tt * RP + c8) * 2) = l4;
+        if constexpr (!SUMMARY) {
+          split8v(qbv, h4, l4);
+          *(uint4 *)(QB + (tt * RP + c8) * 2) = h4;
+          *(uint4 *)(QB + KB_LO + (tt * RP + c8) * 2) = l4;
+        }
       }
       if (tt == 0) {
         *(float4 *)(EC + c8) = make_float4(__builtin_amdgcn_exp2f(gc8[0]), __builtin_amdgcn_exp2f(gc8[1]),
@@ -4739,7 +4772,7 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
     // channels per lane (four lanes per pair) with the exact pairwise decays
     // from the raw rows; P's diagonal from q_t . k_t
     if (pairwise) {
-      for (int task = tid; task < 4 * NPAIR + C; task += NT) {
+      for (int task = tid; task < 4 * NPAIR + (SUMMARY ? 0 : C); task += NT) {
         if (task < 4 * NPAIR) {
           const int p = task >> 2, part = task & 3;
           const int t = pair_t[p], s = pair_s[p];
@@ -4750,7 +4783,7 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
             const int c = cb + 8 * m;
             float kt[8], qt[8], ks[8];
             bf8(*(const uint4 *)(KB + (t * RP + c) * 2), kt);
-            bf8(*(const uint4 *)(QB + (t * RP + c) * 2), qt);
+            if (!SUMMARY) bf8(*(const uint4 *)(QB + (t * RP + c) * 2), qt);
             bf8(*(const uint4 *)(KB + (s * RP + c) * 2), ks);
             const float4 ga0 = *(const float4 *)(G + t * GP + c), ga1 = *(const float4 *)(G + t * GP + c + 4);
             const float4 gb0 = *(const float4 *)(G + s * GP + c), gb1 = *(const float4 *)(G + s * GP + c + 4);
@@ -4760,7 +4793,7 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
             for (int e = 0; e < 8; e++) {
               const float kse = ks[e] * __builtin_amdgcn_exp2f(dg[e]);
               a = fmaf(kt[e], kse, a);
-              pp = fmaf(qt[e], kse, pp);
+              if (!SUMMARY) pp = fmaf(qt[e], kse, pp);
             }
           }
           a += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(a), 0xB1, 0xF, 0xF, false));   // lane ^ 1
@@ -4776,10 +4809,12 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
               ((__bf16 *)M)[(t - 16) * PP + s] = hi;
               ((__bf16 *)M)[16 * PP + (t - 16) * PP + s] = (__bf16)(-av - (float)hi);
             }
-            const float pv = (sm[SM_NQ * C + t] * nks) * pp;
-            const __bf16 hi = (__bf16)pv;
-            ((__bf16 *)PM)[t * PP + s] = hi;
-            ((__bf16 *)PM)[C * PP + t * PP + s] = (__bf16)(pv - (float)hi);
+            if constexpr (!SUMMARY) {
+              const float pv = (sm[SM_NQ * C + t] * nks) * pp;
+              const __bf16 hi = (__bf16)pv;
+              ((__bf16 *)PM)[t * PP + s] = hi;
+              ((__bf16 *)PM)[C * PP + t * PP + s] = (__bf16)(pv - (float)hi);
+            }
           }
         } else {
           const int t = task - 4 * NPAIR;
@@ -4806,7 +4841,7 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
     // growing and the decaying factors: A_ts = beta_t nk_t (k_t e^{G_t -
     // G_C}) . (nk_s k_s e^{G_C - G_s}) for s < t, P_ts = nq_t (q_t e^{G_t -
     // G_C}) . (nk_s k_s e^{G_C - G_s}) for s <= t (zero above)
-    if (!pairwise && w < 6) {
+    if (!pairwise && w < (SUMMARY ? 3 : 6)) {
       const int blk = w < 3 ? w : w - 3;
       const int ti = blk == 0 ? 0 : 1, si = blk == 2 ? 1 : 0;
       const uint8_t *X = w < 3 ? KB : QB;
@@ -4846,64 +4881,105 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
       }
     }
     // ---- K S0 and Q S0 for this wave's columns, two 16-token tiles
-    bf16x8 sh[4], sl[4];
-#pragma unroll
-    for (int kc = 0; kc < 4; kc++) pf::split8(S[2 * kc], S[2 * kc + 1], sh[kc], sl[kc]);
     f32x4 R[2], oq[2];
-    // key-slot blocks outermost: the four accumulators (k and q, two token
-    // tiles) are independent, and each product pass runs over all four
-    f32x4 ak[2], aq[2];
+    // K S alone, of either state: R_t = beta_t (v_t - (nk k e^G)_t S), or with v = 0
+    auto ks_only = [&](const f32x4 (&X)[8], bool with_v) {
+      bf16x8 xh[4], xl[4];
 #pragma unroll
-    for (int tb = 0; tb < 2; tb++) ak[tb] = aq[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int kc = 0; kc < 4; kc++) pf::split8(X[2 * kc], X[2 * kc + 1], xh[kc], xl[kc]);
+      f32x4 ak[2];
 #pragma unroll
-    for (int kc = 0; kc < 4; kc++) {
-      bf16x8 kh[2], kl[2], qh[2], ql[2];
+      for (int tb = 0; tb < 2; tb++) ak[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int tb = 0; tb < 2; tb++) {
-        const int o = ((16 * tb + c16) * RP + 32 * kc + 8 * q4) * 2;
-        kh[tb] = pf::ld8(KG, o);
-        kl[tb] = pf::ld8(KG, KB_LO + o);
-        qh[tb] = pf::ld8(QG, o);
-        ql[tb] = pf::ld8(QG, KB_LO + o);
+      for (int kc = 0; kc < 4; kc++) {
+        bf16x8 kh[2], kl[2];
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++) {
+          const int o = ((16 * tb + c16) * RP + 32 * kc + 8 * q4) * 2;
+          kh[tb] = pf::ld8(KG, o);
+          kl[tb] = pf::ld8(KG, KB_LO + o);
+        }
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++) ak[tb] = pf::mfma(kh[tb], xh[kc], ak[tb]);
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++) ak[tb] = pf::mfma(kh[tb], xl[kc], ak[tb]);
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++) ak[tb] = pf::mfma(kl[tb], xh[kc], ak[tb]);
       }
 #pragma unroll
       for (int tb = 0; tb < 2; tb++) {
-        ak[tb] = pf::mfma(kh[tb], sh[kc], ak[tb]);
-        aq[tb] = pf::mfma(sh[kc], qh[tb], aq[tb]);
+        const pf::tr4_t vr = pf::col4(VR, 16 * tb + 4 * q4, jw, c16);
+        const float4 be = *(const float4 *)(sm + SM_BETA * C + 16 * tb + 4 * q4);
+        const float be4[4] = {be.x, be.y, be.z, be.w};
+#pragma unroll
+        for (int r = 0; r < 4; r++) R[tb][r] = be4[r] * ((with_v ? pf::bf2f((uint16_t)vr[r]) : 0.0f) - ak[tb][r]);
+      }
+    };
+    if constexpr (SUMMARY) {
+      ks_only(S, true);
+    } else {
+      bf16x8 sh[4], sl[4];
+#pragma unroll
+      for (int kc = 0; kc < 4; kc++) pf::split8(S[2 * kc], S[2 * kc + 1], sh[kc], sl[kc]);
+      // key-slot blocks outermost: the four accumulators (k and q, two token
+      // tiles) are independent, and each product pass runs over all four
+      f32x4 ak[2], aq[2];
+#pragma unroll
+      for (int tb = 0; tb < 2; tb++) ak[tb] = aq[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kc = 0; kc < 4; kc++) {
+        bf16x8 kh[2], kl[2], qh[2], ql[2];
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++) {
+          const int o = ((16 * tb + c16) * RP + 32 * kc + 8 * q4) * 2;
+          kh[tb] = pf::ld8(KG, o);
+          kl[tb] = pf::ld8(KG, KB_LO + o);
+          qh[tb] = pf::ld8(QG, o);
+          ql[tb] = pf::ld8(QG, KB_LO + o);
+        }
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++) {
+          ak[tb] = pf::mfma(kh[tb], sh[kc], ak[tb]);
+          aq[tb] = pf::mfma(sh[kc], qh[tb], aq[tb]);
+        }
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++) {
+          ak[tb] = pf::mfma(kh[tb], sl[kc], ak[tb]);
+          aq[tb] = pf::mfma(sl[kc], qh[tb], aq[tb]);
+        }
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++) {
+          ak[tb] = pf::mfma(kl[tb], sh[kc], ak[tb]);
+          aq[tb] = pf::mfma(sh[kc], ql[tb], aq[tb]);
+        }
       }
 #pragma unroll
       for (int tb = 0; tb < 2; tb++) {
-        ak[tb] = pf::mfma(kh[tb], sl[kc], ak[tb]);
-        aq[tb] = pf::mfma(sl[kc], qh[tb], aq[tb]);
+        // R_t = beta_t (v_t - (nk k e^G)_t S0), tokens 16 tb + 4 q4 .. + 3, column jw + c16
+        const pf::tr4_t vr = pf::col4(VR, 16 * tb + 4 * q4, jw, c16);
+        const float4 be = *(const float4 *)(sm + SM_BETA * C + 16 * tb + 4 * q4);
+        const float be4[4] = {be.x, be.y, be.z, be.w};
+#pragma unroll
+        for (int r = 0; r < 4; r++) R[tb][r] = be4[r] * (pf::bf2f((uint16_t)vr[r]) - ak[tb][r]);
+        oq[tb] = aq[tb];  // O^T first term: column 4 q4 + r, token 16 tb + c16
       }
-#pragma unroll
-      for (int tb = 0; tb < 2; tb++) {
-        ak[tb] = pf::mfma(kl[tb], sh[kc], ak[tb]);
-        aq[tb] = pf::mfma(sh[kc], ql[tb], aq[tb]);
-      }
-    }
-#pragma unroll
-    for (int tb = 0; tb < 2; tb++) {
-      // R_t = beta_t (v_t - (nk k e^G)_t S0), tokens 16 tb + 4 q4 .. + 3, column jw + c16
-      const pf::tr4_t vr = pf::col4(VR, 16 * tb + 4 * q4, jw, c16);
-      const float4 be = *(const float4 *)(sm + SM_BETA * C + 16 * tb + 4 * q4);
-      const float be4[4] = {be.x, be.y, be.z, be.w};
-#pragma unroll
-      for (int r = 0; r < 4; r++) R[tb][r] = be4[r] * (pf::bf2f((uint16_t)vr[r]) - ak[tb][r]);
-      oq[tb] = aq[tb];  // O^T first term: column 4 q4 + r, token 16 tb + c16
     }
     pf::lds_barrier();
     // ---- (I + A) Delta = R by blocks: Delta_0 from block 0, then block 1's
     // right-hand side less A10 Delta_0 (M holds -A10); O^T += Delta^T P^T;
     // S <- diag(e^{G_C}) S0 + Kd^T Delta over the 32 tokens
-    const f32x4 d0 = block_solve(A, 0, 0, q4, R[0]);
-    bf16x4 d0h, d0l;
-    pf::split4x(d0, d0h, d0l);
-    const f32x4 d1 = block_solve(A, 16, 16, q4, mm16(M, (c16 * PP + 4 * q4) * 2, MLO, d0h, d0l, R[1]));
-    bf16x4 d1h, d1l;
-    pf::split4x(d1, d1h, d1l);
+    f32x4 d0, d1;
+    bf16x4 d0h, d0l, d1h, d1l;
+    auto solve = [&]() {
+      d0 = block_solve(A, 0, 0, q4, R[0]);
+      pf::split4x(d0, d0h, d0l);
+      if (SUMMARY) __builtin_amdgcn_sched_barrier(0);  // block 1's rows of A after block 0's: 64 registers each
+      d1 = block_solve(A, 16, 16, q4, mm16(M, (c16 * PP + 4 * q4) * 2, MLO, d0h, d0l, R[1]));
+      pf::split4x(d1, d1h, d1l);
+    };
+    solve();
 #pragma unroll
-    for (int tb = 0; tb < 2; tb++) {
+    for (int tb = 0; tb < (SUMMARY ? 0 : 2); tb++) {
       // rows of P for tokens 16 tb + c16: the blocks of source tokens 0-15 and (tb = 1) 16-31
       const int o = ((16 * tb + c16) * PP + 4 * q4) * 2;
       f32x4 acc = oq[tb];
@@ -4916,7 +4992,7 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
         store4(D.out, D.out_dtype, at, o4);
       }
     }
-    {
+    auto state_update = [&](f32x4 (&S)[8]) {
       bf16x8 eh, el;
       pf::split8(d0, d1, eh, el);  // the 32 tokens in the permuted slot order (pcol)
       // four row tiles at a time: their loads first, then each product pass
@@ -4944,6 +5020,17 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
 #pragma unroll
         for (int dt = d4; dt < d4 + 4; dt++) S[dt] = pf::mfma(kl[dt - d4], eh, S[dt]);
       }
+    };
+    state_update(S);
+    if constexpr (SUMMARY) {
+      if (trans) {
+        // M's columns after E's, not beside them (registers); before the
+        // next chunk's staging, which rewrites beta
+        __builtin_amdgcn_sched_barrier(0);
+        ks_only(MS, false);
+        solve();
+        state_update(MS);
+      }
     }
     // The next chunk's staging, issued behind the state update's products
     // (its exponentials and scan run while they do): its rows, norms, beta
@@ -4965,6 +5052,16 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
           for (int r = 0; r < 4; r++) dst[(int64_t)(16 * dt + 4 * q4 + r) * KV] = S[dt][r];
       }
     }
+  }
+  if constexpr (SUMMARY) {
+    const int64_t at = ((int64_t)sg.slot * H + h) * KV * KV + jw + c16;
+#pragma unroll
+    for (int dt = 0; dt < 8; dt++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        D.seg_state[at + (int64_t)(16 * dt + 4 * q4 + r) * KV] = S[dt][r];
+        if (trans) D.seg_trans[at + (int64_t)(16 * dt + 4 * q4 + r) * KV] = MS[dt][r];
+      }
   }
 }
 
@@ -5990,7 +6087,6 @@ int sq_create_cu_stream(int32_t device, int32_t cus, void **stream, int32_t *act
 int sq_prefill_plan(const sq_pool *pool, const int32_t *cu, int64_t batch, int32_t cus, sq_prefill_segments *out) {
   if (!pool || !cu || !out || batch < 0) return fail(SQ_EINVAL, "prefill plan: null argument or negative batch");
   *out = sq_prefill_segments{0, 0, 0, nullptr};
-  if (pool->kda) return 0;
   if (cus <= 0) {
     int dev = 0, n = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -6006,9 +6102,12 @@ int sq_prefill_plan(const sq_pool *pool, const int32_t *cu, int64_t batch, int32
   // every segment's summary and full pass take 7.9 + 7.7 a chunk (256
   // workgroups) over longest / P tokens, and the combine 2.5 a segment.
   // (B = 1, T = 8192, 32 heads: 785 us whole, 127 + 125 + 20 us in 8
-  // segments.)  A split that saves less than 15% is not taken.
-  const double whole_chunk = 6.1, split_chunk = 15.6, step = 2.5, extra = 8.0;
-  const int64_t C = pf::PC;
+  // segments.)  KDA, per 32-token chunk: 8.2 whole, 9.5 + 9.1 split (three
+  // sequences of 3001, 1456 and 2411 tokens, 32 heads: 771 us whole, 304 +
+  // 292 + 15 us in 3 segments).  A split that saves less than 15% is not
+  // taken.
+  const double whole_chunk = pool->kda ? 8.2 : 6.1, split_chunk = pool->kda ? 18.6 : 15.6, step = 2.5, extra = 8.0;
+  const int64_t C = pool->kda ? kc::C : pf::PC;
   int64_t longest = 0;
   for (int64_t b = 0; b < batch; b++) longest = cu[b + 1] - cu[b] > longest ? cu[b + 1] - cu[b] : longest;
   double best = .85 * whole_chunk * (double)((longest + C - 1) / C);
@@ -6073,7 +6172,7 @@ int sq_prefill_split(const sq_pool *pool, const sq_prefill_args *a, const sq_pre
   const bool split = sg && sg->tokens > 0;
   if (split) {
     const int64_t state = (int64_t)pool->heads * 128 * 128 * (int64_t)sizeof(float);
-    if (pool->kda || sg->tokens % pf::PC || sg->count < 2 || sg->count > 16384 || a->batch > 65535 ||
+    if (sg->tokens % (pool->kda ? kc::C : pf::PC) || sg->count < 2 || sg->count > 16384 || a->batch > 65535 ||
         pool->heads > 65535)
       return fail(SQ_EINVAL, "prefill: segments must be whole chunks, two or more a sequence");
     if (!sg->workspace || ((uintptr_t)sg->workspace & 15) || sg->workspace_bytes < 2 * state * a->batch ||
@@ -6137,35 +6236,27 @@ int sq_prefill_split(const sq_pool *pool, const sq_prefill_args *a, const sq_pre
   D.seg = split ? sg->tokens : 0;
   D.seg_state = split ? (float *)sg->workspace : nullptr;
   D.seg_trans = split ? D.seg_state + sg->workspace_bytes / (2 * sizeof(float)) : nullptr;
-  if (pool->kda) {
-    hipError_t e = hipFuncSetAttribute((const void *)kc::kda_chunk_kernel,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, kc::LDS_BYTES);
-    if (e != hipSuccess) return fail((int)e, "prefill: cannot raise the KDA kernel's LDS limit");
-    if (a->events && (e = hipEventRecord((hipEvent_t)a->events[0], st)) != hipSuccess)
-      return fail((int)e, "prefill: hipEventRecord failed");
-    hipLaunchKernelGGL(kc::kda_chunk_kernel, dim3((unsigned)(a->batch * H)), dim3(kc::NT), kc::LDS_BYTES, st, D);
-    rc = check_launch("kda_chunk_kernel");
-  } else {
-    hipError_t e = hipFuncSetAttribute((const void *)pf::prefill_kernel<false>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, pf::LDS_BYTES);
-    if (e == hipSuccess && split)
-      e = hipFuncSetAttribute((const void *)pf::prefill_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              pf::LDS_BYTES);
-    if (e != hipSuccess) return fail((int)e, "prefill: cannot raise the kernel's LDS limit");
-    if (a->events && (e = hipEventRecord((hipEvent_t)a->events[0], st)) != hipSuccess)
-      return fail((int)e, "prefill: hipEventRecord failed");
-    const unsigned tiles = (unsigned)(a->batch * H), count = split ? (unsigned)sg->count : 1u;
-    if (split) {
-      hipLaunchKernelGGL(pf::prefill_kernel<true>, dim3(tiles, count - 1), dim3(pf::NT), pf::LDS_BYTES, st, D);
-      if ((rc = check_launch("prefill_kernel (segment summaries)"))) return rc;
-      if (count > 2) {
-        hipLaunchKernelGGL(pf::segment_combine_kernel, dim3(tiles, 8), dim3(pf::NT), 0, st, D);
-        if ((rc = check_launch("segment_combine_kernel"))) return rc;
-      }
+  const unsigned tiles = (unsigned)(a->batch * H), count = split ? (unsigned)sg->count : 1u;
+  const auto whole = pool->kda ? kc::kda_chunk_kernel<false> : pf::prefill_kernel<false>;
+  const auto summary = pool->kda ? kc::kda_chunk_kernel<true> : pf::prefill_kernel<true>;
+  const int lds = pool->kda ? kc::LDS_BYTES : pf::LDS_BYTES;
+  static_assert(kc::NT == pf::NT, "one launch shape for both recurrence kernels");
+  hipError_t e = hipFuncSetAttribute((const void *)whole, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e == hipSuccess && split)
+    e = hipFuncSetAttribute((const void *)summary, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return fail((int)e, "prefill: cannot raise the kernel's LDS limit");
+  if (a->events && (e = hipEventRecord((hipEvent_t)a->events[0], st)) != hipSuccess)
+    return fail((int)e, "prefill: hipEventRecord failed");
+  if (split) {
+    hipLaunchKernelGGL(summary, dim3(tiles, count - 1), dim3(pf::NT), lds, st, D);
+    if ((rc = check_launch("segment summaries"))) return rc;
+    if (count > 2) {
+      hipLaunchKernelGGL(pf::segment_combine_kernel, dim3(tiles, 8), dim3(pf::NT), 0, st, D);
+      if ((rc = check_launch("segment_combine_kernel"))) return rc;
     }
-    hipLaunchKernelGGL(pf::prefill_kernel<false>, dim3(tiles, count), dim3(pf::NT), pf::LDS_BYTES, st, D);
-    rc = check_launch("prefill_kernel");
   }
+  hipLaunchKernelGGL(whole, dim3(tiles, count), dim3(pf::NT), lds, st, D);
+  rc = check_launch(pool->kda ? "kda_chunk_kernel" : "prefill_kernel");
   if (rc) return rc;
   if (a->events) {
     const hipError_t e = hipEventRecord((hipEvent_t)a->events[1], st);

@@ -79,13 +79,15 @@ LENS = [640, 0, 128, 129, 1, 333]
 MARKS = [[128, 640], [0, 0], [64, 128], [128, 129], [1, 0], [130, 333]]
 
 
-@pytest.mark.parametrize("arch,tokens", [("gdn", 64), ("gdn", 128), ("gdn", 320)])
+@pytest.mark.parametrize("arch,tokens", [("gdn", 64), ("gdn", 128), ("gdn", 320), ("kda", 32), ("kda", 96),
+                                         ("kda", 320)])
 def test_segments_against_the_recurrence(arch, tokens, monkeypatch):
     print(f"case {arch} tokens={tokens}", flush=True)
     _case(arch, LENS, MARKS, tokens, monkeypatch)
 
 
-@pytest.mark.parametrize("arch,storage", [("gdn", "packed"), ("gdn", "byte")])
+@pytest.mark.parametrize("arch,storage", [("gdn", "packed"), ("gdn", "byte"), ("kda", "packed"),
+                                          ("kda", "byte")])
 def test_planned_segments_against_the_recurrence(arch, storage, monkeypatch):
     """The plan's own choice, offsets on the device, byte pages (dense
     initial states) and packed ones."""

@@ -21,12 +21,13 @@ def test_whole_sequences(lens, heads):
     assert (plan.tokens, plan.count, plan.workspace_bytes) == (0, 0, 0)
 
 
+@pytest.mark.parametrize("arch", ["gdn", "kda"])
 @pytest.mark.parametrize("lens,heads", [([8192], 32), ([8192], 8), ([8192], 4), ([3000, 17, 0, 900], 16), ([6972, 6972], 16),
                                         ([4096, 1], 32), ([65536], 1)])
-def test_segments_cover_the_sequences_and_fit_the_device(lens, heads):
-    plan = _plan(lens, heads)
+def test_segments_cover_the_sequences_and_fit_the_device(lens, heads, arch):
+    plan = _plan(lens, heads, arch)
     n = [-(-t // plan.tokens) for t in lens]
-    assert plan.tokens % 64 == 0 and plan.count == max(n) >= 2
+    assert plan.tokens % (64 if arch == "gdn" else 32) == 0 and plan.count == max(n) >= 2
     assert sum(n) * heads <= CUS and sum(max(0, x - 1) for x in n) * heads <= CUS
     # every segment's workspace slot, t0 / tokens + b + s, is its own and inside the workspace
     starts = np.concatenate([[0], np.cumsum(lens)])[:-1]
