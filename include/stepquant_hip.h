@@ -289,6 +289,17 @@ int sq_copy_slots(const sq_pool *pool, const void *src, const void *dst, int32_t
                   int64_t n, uint8_t *temp, void *stream);
 
 /*
+ * The same copy of at most SQ_COPY_DIRECT_PAGES pages without `temp`: one
+ * kernel holds each byte range of all the pages between reading and writing
+ * it.  Page sizes must be even and the pool 16-byte aligned (SQ_EINVAL
+ * otherwise, and above that count).  Safe under capture and on any number
+ * of streams.
+ */
+#define SQ_COPY_DIRECT_PAGES 256
+int sq_copy_slots_direct(const sq_pool *pool, const void *src, const void *dst, int32_t slots_dtype, int64_t n,
+                         void *stream);
+
+/*
  * No counterpart in the reference.  sq_copy_slots without the `temp`
  * argument, for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid

@@ -5082,6 +5082,85 @@ __global__ void clear_kernel(uint8_t *data, int64_t page_bytes, int64_t num_slot
     p[e] = 0;
 }
 
+// Pages src[i] -> dst[i], i < n, all read before any is written: the same byte
+// range of every page is one workgroup's, which holds it (n * LR windows of
+// 16 bytes, at most 64 KB: two workgroups per CU) between its loads and its
+// stores, so overlapping lists behave as a gather followed by a scatter with
+// two passes over memory instead of four and no staging buffer.  LR lanes
+// take a row's windows.  ALIGNED (page bytes and base multiples of 16): a
+// range is 16 LR bytes and stays in registers.  Otherwise (even sizes): 16
+// LR - 16 bytes, read in aligned 16-byte windows into LDS and written in the
+// destination's windows, edges in 2-byte units.  A pair whose source or
+// destination lies outside the pool is skipped; negative indices wrap.
+// Bound by HBM: 64 pages of 409,600 B in 9.7 us (5.4 TB/s read and written),
+// 75 us as a byte-wise gather and scatter.
+constexpr int COPY_WINDOWS = 4096;  // windows of a workgroup: 16 a thread
+constexpr int COPY_PAGES = SQ_COPY_DIRECT_PAGES;  // LR >= 16
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// PER: windows a thread holds (rows threadIdx.x / LR + it 256 / LR).  Their
+// loads are unconditional, from rows and windows clamped into the copy, so
+// that they go out back to back.
+template <bool ALIGNED, int PER>
+__global__ __launch_bounds__(256) void copy_kernel(uint8_t *data, int64_t page_bytes, int64_t num_slots,
+                                                   const void *src, const void *dst, int dtype, int n, int lr_log) {
+  extern __shared__ __align__(16) uint8_t smem[];  // !ALIGNED: [rows][LR] windows
+  __shared__ int64_t from[COPY_PAGES], to[COPY_PAGES];  // byte offsets of the pages; to < 0: skipped
+  const int LR = 1 << lr_log, lane = threadIdx.x & (LR - 1), row0 = threadIdx.x >> lr_log, rows = 256 >> lr_log;
+  const int64_t range = 16 * (ALIGNED ? LR : LR - 1), p0 = blockIdx.x * range;
+  const int bytes = (int)(p0 + range < page_bytes ? range : page_bytes - p0);
+  if ((int)threadIdx.x < n) {
+    int64_t s = load_slot(src, dtype, threadIdx.x), d = load_slot(dst, dtype, threadIdx.x);
+    if (s < 0) s += num_slots;
+    if (d < 0) d += num_slots;
+    const bool live = s >= 0 && s < num_slots && d >= 0 && d < num_slots;
+    from[threadIdx.x] = live ? s * page_bytes : 0;
+    to[threadIdx.x] = live ? d * page_bytes : -1;
+  }
+  __syncthreads();
+  u32x4 x[PER];
+#pragma unroll
+  for (int it = 0; it < PER; it++) {
+    const int r = row0 + it * rows;
+    uint8_t *at = data + from[r < n ? r : n - 1] + p0;
+    const int shift = ALIGNED ? 0 : (int)((uintptr_t)at & 15), last = (shift + bytes - 1) & ~15;
+    x[it] = *(const u32x4 *)(at - shift + (16 * lane < last ? 16 * lane : last));
+  }
+  if (!ALIGNED) {
+#pragma unroll
+    for (int it = 0; it < PER; it++) ((u32x4 *)smem)[(row0 + it * rows) * LR + lane] = x[it];
+  }
+  // every load of the workgroup has arrived before its first store
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < PER; it++) {
+    const int r = row0 + it * rows;
+    if (r >= n || to[r] < 0) continue;
+    uint8_t *at = data + to[r] + p0;
+    if (ALIGNED) {
+      if (16 * lane < bytes) *(u32x4 *)(at + 16 * lane) = x[it];
+      continue;
+    }
+    // byte b of the range at row + b; this lane's destination window starts at byte b0
+    const uint8_t *row = smem + 16 * (r * LR) + (int)((uintptr_t)(data + from[r] + p0) & 15);
+    const int b0 = 16 * lane - (int)((uintptr_t)at & 15);
+    uint8_t *out = at + b0;
+    if (b0 >= 0 && b0 + 16 <= bytes) {
+      uint32_t w[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) w[u] = *(const uint16_t *)(row + b0 + 2 * u);
+      *(u32x4 *)out = u32x4{w[0] | w[1] << 16, w[2] | w[3] << 16, w[4] | w[5] << 16, w[6] | w[7] << 16};
+    } else {
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        const int b = b0 + 2 * u;
+        if (b >= 0 && b + 2 <= bytes) *(uint16_t *)(out + 2 * u) = *(const uint16_t *)(row + b);
+      }
+    }
+  }
+}
+
 // Pages src[y] -> temp[y] (scatter == 0) or temp[y] -> dst[y] (scatter == 1).
 // Negative indices wrap like Python; a pair whose source or destination
 // lies outside the pool is skipped in both passes, so a destination never
@@ -5806,8 +5885,29 @@ int static_scratch(uint8_t **out) {
   return 0;
 }
 
+bool copy_is_direct(const sq_pool *pool, int64_t n) {
+  return n <= COPY_PAGES && pool->page_bytes > 0 && pool->page_bytes % 2 == 0 && ((uintptr_t)pool->data & 15) == 0;
+}
+
+// temp may be NULL for lists that copy_kernel takes
 int launch_copy(const sq_pool *pool, const void *src, const void *dst, int32_t slots_dtype, int64_t n,
                 uint8_t *temp, hipStream_t stream) {
+  if (copy_is_direct(pool, n)) {
+    const int lr_log = n <= 64 ? 6 : n <= 128 ? 5 : 4;
+    const bool aligned = pool->page_bytes % 16 == 0;
+    const int64_t range = 16 * ((1 << lr_log) - (aligned ? 0 : 1)), blocks = (pool->page_bytes + range - 1) / range;
+    const int per = (int)((n << lr_log) + 255) / 256;  // windows of a thread
+    auto launch = [&](auto kernel, int windows) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), aligned ? 0 : 16 * 256 * windows, stream,
+                         pool->data, pool->page_bytes, pool->num_slots, src, dst, slots_dtype, (int)n, lr_log);
+    };
+    if (blocks < (int64_t)1 << 31) {
+      if (per > 4) launch(aligned ? copy_kernel<true, 16> : copy_kernel<false, 16>, COPY_WINDOWS / 256);
+      else if (per > 1) launch(aligned ? copy_kernel<true, 4> : copy_kernel<false, 4>, 4);
+      else launch(aligned ? copy_kernel<true, 1> : copy_kernel<false, 1>, 1);
+      return check_launch("copy_kernel");
+    }
+  }
   unsigned gx = (unsigned)((pool->page_bytes + 255) / 256);
   if (gx > 1024) gx = 1024;
   hipLaunchKernelGGL(gather_kernel, dim3(gx, (unsigned)n), dim3(256), 0, stream, pool->data,
@@ -6286,6 +6386,15 @@ int sq_copy_slots(const sq_pool *pool, const void *src, const void *dst, int32_t
   if (!src || !dst || !temp || n < 0 || n > 65535) return fail(SQ_EINVAL, "copy: bad arguments");
   if (slots_dtype != SQ_I32 && slots_dtype != SQ_I64) return fail(SQ_EINVAL, "copy: slots dtype");
   return launch_copy(pool, src, dst, slots_dtype, n, temp, (hipStream_t)stream);
+}
+
+int sq_copy_slots_direct(const sq_pool *pool, const void *src, const void *dst, int32_t slots_dtype, int64_t n,
+                         void *stream) {
+  if (!pool || !pool->data) return fail(SQ_EINVAL, "copy_direct: null pool");
+  if (n == 0) return 0;
+  if (!src || !dst || n < 0 || !copy_is_direct(pool, n)) return fail(SQ_EINVAL, "copy_direct: bad arguments");
+  if (slots_dtype != SQ_I32 && slots_dtype != SQ_I64) return fail(SQ_EINVAL, "copy_direct: slots dtype");
+  return launch_copy(pool, src, dst, slots_dtype, n, nullptr, (hipStream_t)stream);
 }
 
 int sq_copy_slots_static(const sq_pool *pool, const void *src, const void *dst, int32_t slots_dtype, int64_t n,

@@ -579,7 +579,10 @@ class PackedStatePool:
         dst = _indices(destination, self.device).to(torch.int64)
         if src.numel() != dst.numel():
             raise ValueError("copy needs as many destination slots as source slots")
-        if src.numel():
+        if 0 < src.numel() <= N.COPY_DIRECT_PAGES and self.page_bytes % 2 == 0:
+            N.check(N.lib().sq_copy_slots_direct(self._desc, N.ptr(src), N.ptr(dst), N.I64, src.numel(),
+                                                 N.stream_handle()), "copy")
+        elif src.numel():
             temp = torch.empty((src.numel(), self.page_bytes), device=self.device, dtype=torch.uint8)
             N.check(N.lib().sq_copy_slots(self._desc, N.ptr(src), N.ptr(dst), N.I64, src.numel(), N.ptr(temp),
                                           N.stream_handle()), "copy")
