@@ -80,9 +80,10 @@ typedef struct sq_pool {
 } sq_pool;
 
 /* sq_pool.flags: the pool qualifies for the K=V=128 uniform-width GDN kernel,
- * or for the K=V=128 KDA kernel */
+ * for the K=V=128 KDA kernel, or (byte storage) for the K=V=128 byte kernel */
 #define SQ_POOL_FAST_GDN128 1
 #define SQ_POOL_FAST_KDA128 2
+#define SQ_POOL_FAST_BYTE128 4
 
 /*
  * Inputs of one decode step (PackedStatePool.step, pool.py:200-282).

@@ -16,7 +16,7 @@ ABI_VERSION = 2
 
 F32, BF16, F16, I32, I64 = 0, 1, 2, 3, 4
 # sq_pool.flags bits (SQ_POOL_FAST_*)
-POOL_FAST_GDN128, POOL_FAST_KDA128 = 1, 2
+POOL_FAST_GDN128, POOL_FAST_KDA128, POOL_FAST_BYTE128 = 1, 2, 4
 _DTYPES = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16, torch.int32: I32, torch.int64: I64}
 
 _P = ctypes.c_void_p

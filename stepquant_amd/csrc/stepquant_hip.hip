@@ -3331,6 +3331,380 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KDA128_WAVE
 }
 
 // =====================================================================
+// Byte pages, K = V = 128, GDN (one width per head) and KDA (per-row widths,
+// FP16 pivot rows): the decode step's three modes.  The operations of the
+// general kernel in its order (IEEE divisions, its fused multiply-adds, its
+// summation trees), so both give the same bits; lane (rg, cg) owns rows
+// rg + 8 r of columns 4 cg .. 4 cg + 3 there and here.  What differs is the
+// way to them.  A head's int8 plane holds value (i, j) at i + 128 j: it is
+// staged by direct global-to-LDS loads, a lane gets its 8 rows of a column
+// from one transposing LDS load (ds_read_b64_tr_b8: of a 16-lane row's 16 x 8
+// bytes, lane l receives byte l % 8 of rows l / 8 + 2 k), new carriers go
+// back as one LDS byte each (the low byte of 1.5 2^23 + z) in a padded
+// plane, and per-row constants are formed once per row instead of by each of
+// its 32 lanes.  Four workgroups per CU (128 registers, 28 KB of LDS).
+// Bound by VALU issue and the dependent phases.  B = 128, 32 heads, GDN@6:
+// readout 30 us and writer 51 us; the general kernel (one LDS byte per value,
+// the tables and divisions in every lane) 74 and 147 us.
+// =====================================================================
+namespace bfast {
+
+using fast::FK;
+using fast::FNT;
+using fast::FV;
+using fast::hw_h2f;
+using fast::rg8_sum;
+using fast::wave_sum;
+
+enum { GDN_INT = 0, GDN_TWO = 1, KDA_ROWS = 2, GDN_PIV = 3 };
+constexpr int CP = FK + 16;     // padded column of the outgoing plane: the 8 column groups of a wave spread over the banks
+constexpr int REDP = FK + 8;    // row pitch of the row sums, for the same reason
+
+struct Lds {
+  uint8_t plane[FV * CP];  // staged plane (pitch 128), then row sums [32][REDP] f32, then the outgoing plane (pitch CP)
+  float2 kq[FK];           // per row: k, q
+  float rt[4][FK];         // per (group, row): r * retention (pivot rows: retention)
+  float4 iu[4][FK];        // per (group, row): 1 / (r' norm), U = w^2 (r' norm)^2, 1 / L, L' = 1 / (1 / L)
+  float wv[FK];
+  int rowpos[FK];  // byte offset of the row's first scale in the page, -1 for pivots
+  int pivpos[FK];  // byte offset of a pivot row's halves
+  int wid[FK];     // KDA: the row's width
+  uint64_t piv[2];
+};
+
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+
+template <int MODE, bool QW4, int KIND>
+__device__ __forceinline__ void body(const PoolDev &P, const StepDev &S, Lds &T, uint8_t *page, int b, int h, int W) {
+#pragma clang fp contract(off)
+  const int tid = threadIdx.x, rg = tid & 7, j0 = 4 * (tid >> 3), wave = tid >> 6, l = tid & 63;
+  const int i = tid & (FK - 1);
+  const int64_t bh = (int64_t)b * P.H + h, hr = (int64_t)h * FK;
+  const int colbase = ld_uniform(P.columns + h), plane = ld_uniform(P.offsets + (int64_t)P.H * FK + h);
+  const int NG = KIND == GDN_TWO ? P.ng : 1;
+  const int g = KIND == GDN_TWO ? (j0 * P.ng) >> 7 : 0;
+  const bool ints = KIND == KDA_ROWS ? colbase >= 0 : KIND != GDN_PIV;  // the head has integer rows
+  // ---- every load of the tile, then the first use
+  uint32_t ch[4] = {0, 0, 0, 0};
+  if (ints) {
+    const uint4 *src = (const uint4 *)(page + plane) + tid;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      __builtin_amdgcn_global_load_lds((fast::gptr_t)(src + FNT * k),
+                                       (fast::lptr_t)(T.plane + 16 * (FNT * k + 64 * wave)), 16, 0, 0);
+#pragma unroll
+    for (int c = 0; c < 4; c++) ch[c] = *(const uint16_t *)(page + colbase + 2 * (j0 + c));
+  }
+  const int width = KIND == KDA_ROWS ? P.bits[hr + i] : W;
+  const int rpos = P.rows[hr + i], ppos = P.offsets[hr + i];
+  const float w = P.impact[hr + i];
+  float kv, qv = 0.0f, gv, bt = 0.0f, vv[4];
+  if (MODE == MODE_WRITE) {
+    kv = S.s_key[bh * FK + i];
+    gv = S.s_decay[bh * FK + i];
+    __builtin_memcpy(vv, S.s_delta + bh * FV + j0, 16);
+  } else {
+    const int hk = (h * S.hk_mul) >> 20;
+    const int64_t qb = (int64_t)b * S.q_stride + (int64_t)hk * FK, kb = (int64_t)b * S.k_stride + (int64_t)hk * FK;
+    const int64_t gi = KIND == KDA_ROWS ? bh * FK + i : bh, di = KIND == KDA_ROWS ? hr + i : h;
+    // every wave reads the whole rows (l, l + 64) for the norms
+    float q2[2], k2[2];
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      q2[e] = QW4 ? ((const float *)S.q)[qb + l + 64 * e] : load_val(S.q, S.qkv_dtype, qb + l + 64 * e);
+      k2[e] = QW4 ? ((const float *)S.k)[kb + l + 64 * e] : load_val(S.k, S.qkv_dtype, kb + l + 64 * e);
+    }
+    load4(S.v, QW4 ? SQ_F32 : S.qkv_dtype, (int64_t)b * S.v_stride + (int64_t)h * FV + j0, vv);
+    gv = load_val(S.g, S.gate_dtype, gi);
+    bt = load_val(S.beta, S.gate_dtype, bh);
+    float dtb = 0.0f, alog = 0.0f;
+    if (S.a_log) {
+      dtb = load_val(S.dt_bias, S.gate_dtype, di);
+      alog = __expf(load_val(S.a_log, S.gate_dtype, h));
+      bt = 1.0f / (1.0f + __expf(-bt));
+    }
+    const float sq = wave_sum(fmaf(q2[1], q2[1], q2[0] * q2[0])), sk = wave_sum(fmaf(k2[1], k2[1], k2[0] * k2[0]));
+    const float nq = S.normalize ? 1.0f / __builtin_sqrtf(sq + 1e-6f) : 1.0f;
+    const float nk = S.normalize ? 1.0f / __builtin_sqrtf(sk + 1e-6f) : 1.0f;
+    qv = ((wave & 1 ? q2[1] : q2[0]) * nq) * S.scale;  // row i = tid mod 128
+    kv = (wave & 1 ? k2[1] : k2[0]) * nk;
+    if (S.a_log) {
+      const float u = gv + dtb;
+      const float sp = u > 20.0f ? u : __logf(1.0f + __expf(u < 20.0f ? u : 20.0f));
+      gv = -alog * sp;
+    }
+    gv = __expf(gv);
+  }
+  if (tid < FK) {
+    T.kq[i] = make_float2(kv, qv);
+    if (MODE == MODE_READ) {
+      S.s_key[bh * FK + i] = kv;
+      S.s_decay[bh * FK + i] = gv;
+    }
+#pragma unroll
+    for (int e = 0; e < (KIND == GDN_TWO ? 4 : 1); e++)
+      if (e < NG) T.rt[e][i] = rpos >= 0 ? h2f(*(const uint16_t *)(page + rpos + 2 * e)) * gv : gv;
+  } else {
+    T.wv[i] = w;
+    T.rowpos[i] = rpos;
+    T.pivpos[i] = ppos;
+    T.wid[i] = width;
+    const uint64_t m = __ballot(width == 16);
+    if (l == 0) T.piv[wave - 2] = m;
+  }
+  __syncthreads();
+  const bool pivots = KIND == KDA_ROWS ? (T.piv[0] | T.piv[1]) != 0 : KIND == GDN_PIV;
+
+  // ---- this lane's values, x = ((r d) c_j) z (pivots: half * d)
+  float x[16][4];
+  float cj[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) cj[c] = h2f(ch[c]);
+  if (ints) {
+    const int i16 = l & 15;
+    const uint8_t *at = T.plane + FK * (8 * (tid >> 4) + 4 * (i16 & 1)) + 8 * (i16 >> 1);
+    uint32_t z[4][4];
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int e = 0; e < 2; e++) {
+        const i32x2 v = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+            (__attribute__((address_space(3))) i32x2 *)(uintptr_t)(fast::lptr_t)(at + FK * c + 64 * e));
+        z[c][2 * e] = (uint32_t)v[0];
+        z[c][2 * e + 1] = (uint32_t)v[1];
+      }
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const float a = T.rt[g][rg + 8 * r];
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+        x[r][c] = (a * cj[c]) * (float)((int)(z[c][r >> 2] << (24 - 8 * (r & 3))) >> 24);
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) x[r][c] = 0.0f;
+  }
+  // rows 8 r .. 8 r + 7 of the pivot mask (workgroup-uniform)
+  auto piv8 = [&](int r) {
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)((T.piv[r >> 3] >> (8 * (r & 7))) & 255u));
+  };
+  if (pivots) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const uint32_t m = piv8(r);
+      if (m && ((m >> rg) & 1u)) {
+        const int row = rg + 8 * r;
+        const uint2 hv = *(const uint2 *)(page + T.pivpos[row] + 2 * j0);
+        const float d = T.rt[0][row];
+        x[r][0] = h2f(hv.x & 0xffffu) * d;
+        x[r][1] = h2f(hv.x >> 16) * d;
+        x[r][2] = h2f(hv.y & 0xffffu) * d;
+        x[r][3] = h2f(hv.y >> 16) * d;
+      }
+    }
+  }
+
+  // values complete here: otherwise their operands stay live beside them
+  auto settle = [&]() {
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) asm volatile("" : "+v"(x[r][c]));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  settle();
+  // ---- delta = beta (v - k^T x); x' = x + k delta; o = q^T x'
+  float delta[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    if (MODE == MODE_WRITE) {
+      delta[c] = vv[c];
+    } else {
+      float s = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 16; r++) s = fmaf(T.kq[rg + 8 * r].x, x[r][c], s);
+      delta[c] = bt * (vv[c] - rg8_sum(s));
+    }
+  }
+  float o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const float2 kq = T.kq[rg + 8 * r];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      x[r][c] = fmaf(kq.x, delta[c], x[r][c]);
+      if (MODE != MODE_WRITE) o[c] = fmaf(kq.y, x[r][c], o[c]);
+    }
+  }
+  if (MODE != MODE_WRITE) {
+#pragma unroll
+    for (int c = 0; c < 4; c++) o[c] = rg8_sum(o[c]);
+    if (rg == 0) {
+      store4(S.out, S.out_dtype, bh * FV + j0, o);
+      if (MODE == MODE_READ) *(float4 *)(S.s_delta + bh * FV + j0) = make_float4(delta[0], delta[1], delta[2], delta[3]);
+    }
+  }
+  if (MODE == MODE_READ) return;
+  settle();
+
+  // ================= requantise =================
+  if (pivots) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const uint32_t m = piv8(r);
+      if (m && ((m >> rg) & 1u)) {
+        uint2 hv;
+        hv.x = f2h(x[r][0]) | (f2h(x[r][1]) << 16);
+        hv.y = f2h(x[r][2]) | (f2h(x[r][3]) << 16);
+        *(uint2 *)(page + T.pivpos[rg + 8 * r] + 2 * j0) = hv;
+      }
+    }
+  }
+  if (!ints) return;
+  __syncthreads();  // the staged plane is read: its space takes the row sums
+  float *red = (float *)T.plane;
+#pragma unroll
+  for (int r = 0; r < 16; r++)
+    red[(tid >> 3) * REDP + rg + 8 * r] = ((fabsf(x[r][0]) + fabsf(x[r][1])) + fabsf(x[r][2])) + fabsf(x[r][3]);
+  __syncthreads();
+  {
+    const int ngsh = KIND == GDN_TWO ? P.ngsh : 0, cgs = 32 >> ngsh;  // column groups of a value group
+    const float ginv = __builtin_amdgcn_ldexpf(1.0f, ngsh - 7);     // 1 / values of a group, a power of two
+    for (int e = tid; e < FK * NG; e += FNT) {
+      const int row = e >> ngsh, gq = e & (NG - 1);
+      const int wd = KIND == KDA_ROWS ? T.wid[row] : W;
+      if (KIND == KDA_ROWS && wd == 16) {  // nothing of a pivot row reaches the column statistics
+        T.iu[gq][row] = make_float4(0.f, 0.f, 0.f, 0.f);
+        continue;
+      }
+      const float *src = red + gq * cgs * REDP + row;
+      float sum = 0.0f;
+#pragma unroll 8
+      for (int q = 0; q < cgs; q++) sum += src[q * REDP];
+      float m = sum * ginv;
+      m = m < 1e-20f ? 1e-20f : m;
+      const float wi = T.wv[row];
+      uint32_t hb;
+      float rn = fp16_scale(__builtin_sqrtf(m / wi), &hb);
+      put_page_half(page, T.rowpos[row] + 2 * gq, hb);
+      rn = rn * (KIND == KDA_ROWS ? (float)(1 << (8 - wd)) : 1.0f);
+      const float iL = KIND == GDN_TWO ? 1.0f / 3.0f : 1.0f / (float)((1 << (wd - 1)) - 1);
+      T.iu[gq][row] = make_float4(1.0f / rn, (wi * wi) * (rn * rn), iL, KIND == GDN_TWO ? 3.0f : 1.0f / iL);
+    }
+  }
+  __syncthreads();
+  const float4 *iul = T.iu[g] + rg;
+  float mx[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const float4 u = iul[8 * r];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      x[r][c] = x[r][c] * u.x;
+      mx[c] = fmaxf(mx[c], fabsf(x[r][c]) * u.z);
+    }
+  }
+  settle();
+  float f[4], c0[4], num[4] = {0.f, 0.f, 0.f, 0.f}, den[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    c0[c] = fp16_scale(fast::rg8_max_nonneg(mx[c]), nullptr);
+    f[c] = 1.0f / c0[c];
+  }
+  // scaled level of a value (unclamped rint for the integer kinds)
+  auto two_level = [](float y) { return (y >= 0.0f ? 1.0f : -1.0f) * (fabsf(y) >= 2.0f ? 3.0f : 1.0f); };
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const float4 u = iul[8 * r];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const float y = x[r][c] * f[c];
+      const float z = KIND == GDN_TWO ? two_level(y) : __builtin_amdgcn_fmed3f(__builtin_rintf(y), -u.w, u.w);
+      const float t = u.y * z;
+      num[c] = fmaf(t, x[r][c], num[c]);
+      den[c] = fmaf(t, z, den[c]);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const float n = rg8_sum(num[c]), d = rg8_sum(den[c]);
+    const float dc = d < 1e-30f ? 1e-30f : d;
+    uint32_t hb;
+    const float cc = fp16_scale(d > 0.0f ? n / dc : c0[c], &hb);
+    f[c] = 1.0f / cc;
+    if (rg == 0) put_page_half(page, colbase + 2 * (j0 + c), hb);
+  }
+  settle();
+  // ---- final carriers: 1.5 2^23 + n holds the integer n in its low bits
+  constexpr float MAGIC = 12582912.0f;
+  const float Lh = (float)((1 << (W - 1)) - 1);  // GDN_INT: the head's level count
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const int row = rg + 8 * r, wd = KIND == KDA_ROWS ? T.wid[row] : W;
+    const float L = KIND == KDA_ROWS ? (float)((1 << ((wd < 8 ? wd : 8) - 1)) - 1) : Lh;
+    const float nm = KIND == KDA_ROWS ? (float)(1 << (8 - (wd < 8 ? wd : 8))) : 1.0f;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const float y = x[r][c] * f[c];
+      float z;
+      if (KIND == GDN_TWO) z = two_level(y) + MAGIC;
+      else if (KIND == GDN_INT) z = __builtin_amdgcn_fmed3f(y + MAGIC, MAGIC - Lh, MAGIC + Lh);
+      else z = fmaf(__builtin_amdgcn_fmed3f(__builtin_rintf(y), -L, L), nm, MAGIC);
+      T.plane[(j0 + c) * CP + row] = (uint8_t)__float_as_uint(z);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const int e = tid + FNT * k, col = e >> 3, r0 = 16 * (e & 7);
+    uint4 *dst = (uint4 *)(page + plane) + e;
+    uint4 v = *(const uint4 *)(T.plane + col * CP + r0);
+    if (KIND == KDA_ROWS && pivots) {  // the plane's bytes of pivot rows stay as they are
+      const uint32_t m16 = (uint32_t)(T.piv[r0 >> 6] >> (r0 & 63)) & 0xffffu;
+      if (m16) {
+        const uint4 old = *dst;
+        const uint32_t was[4] = {old.x, old.y, old.z, old.w};
+        uint32_t now[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const uint32_t keep = ((((m16 >> (4 * q)) & 15u) * 0x00204081u) & 0x01010101u) * 255u;
+          now[q] = (was[q] & keep) | (now[q] & ~keep);
+        }
+        v = make_uint4(now[0], now[1], now[2], now[3]);
+      }
+    }
+    *dst = v;
+  }
+}
+
+}  // namespace bfast
+
+template <int MODE, bool QW4, bool KDA>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void byte128_kernel(PoolDev P, StepDev S) {
+  __shared__ bfast::Lds T;
+  const int b = blockIdx.y;
+  const int h = P.hrot ? (int)((blockIdx.x + blockIdx.y) & (unsigned)P.hrot) : (int)blockIdx.x;
+  int64_t slot;
+  if (MODE == MODE_WRITE) slot = ld_uniform(S.s_slots + b);
+  else slot = load_slot_uniform(S.slots, S.slots_dtype, b);
+  const int W = ld_uniform(P.bits + (int64_t)h * fast::FK);  // GDN: the head's width
+  if (MODE == MODE_READ && h == 0 && threadIdx.x == 0) S.s_slots[b] = slot;
+  if (slot <= 0 || slot >= P.num_slots) {
+    if (MODE != MODE_WRITE)
+      for (int j = threadIdx.x; j < fast::FV; j += 256)
+        store_val(S.out, S.out_dtype, ((int64_t)b * P.H + h) * fast::FV + j, 0.0f);
+    return;
+  }
+  uint8_t *page = P.data + slot * P.page_bytes;
+  if constexpr (KDA) bfast::body<MODE, QW4, bfast::KDA_ROWS>(P, S, T, page, b, h, 8);
+  else if (W == 16) bfast::body<MODE, QW4, bfast::GDN_PIV>(P, S, T, page, b, h, W);
+  else if (W == 2) bfast::body<MODE, QW4, bfast::GDN_TWO>(P, S, T, page, b, h, W);
+  else bfast::body<MODE, QW4, bfast::GDN_INT>(P, S, T, page, b, h, W);
+}
+
+// =====================================================================
 // Chunked GDN prefill, K = V = 128, chunks of 64 tokens, bf16 MFMA
 // (v_mfma_f32_16x16x32_bf16) with fp32 accumulation.
 //
@@ -5654,7 +6028,7 @@ PoolDev to_dev(const sq_pool *p) {
   d.kda = p->kda;
   d.stage = (p->max_code_bytes + 47) & ~15;
   d.rstage = (p->max_row_bytes + 15) & ~15;
-  d.fast = p->flags & (SQ_POOL_FAST_GDN128 | SQ_POOL_FAST_KDA128);
+  d.fast = p->flags & (SQ_POOL_FAST_GDN128 | SQ_POOL_FAST_KDA128 | SQ_POOL_FAST_BYTE128);
   d.storage = p->storage;
   d.hrot = (p->heads & (p->heads - 1)) == 0 ? p->heads - 1 : 0;
   return d;
@@ -5669,7 +6043,7 @@ int launch_step_mode(const sq_pool *pool, StepDev sd, int64_t batch, hipStream_t
   // head h as (h * hk_mul) >> 20 (exact for h * (H / HK) < 2^20): larger shapes
   // run on the general kernels below.
   if (pool->heads > 1024 || batch > 65535) pd.fast = 0;
-  if (pd.fast & (SQ_POOL_FAST_GDN128 | SQ_POOL_FAST_KDA128)) {
+  if (pd.fast) {
     const int ratio = sd.HK > 0 ? pool->heads / sd.HK : 1;
     sd.hk_mul = ((1 << 20) + ratio - 1) / ratio;
   }
@@ -5692,6 +6066,16 @@ int launch_step_mode(const sq_pool *pool, StepDev sd, int64_t batch, hipStream_t
     return check_launch("kda128_kernel (decode)");
   }
   if constexpr (MODE != MODE_DECODE) {
+    if ((pd.fast & SQ_POOL_FAST_BYTE128) && ((uintptr_t)pool->data & 15) == 0) {
+      const dim3 grid((unsigned)pool->heads, (unsigned)batch);
+      const bool f32 = MODE == MODE_WRITE || sd.qkv_dtype == SQ_F32;
+      constexpr bool W32 = MODE == MODE_WRITE;
+      if (pool->kda && f32) hipLaunchKernelGGL((byte128_kernel<MODE, true, true>), grid, dim3(256), 0, st, pd, sd);
+      else if (pool->kda) hipLaunchKernelGGL((byte128_kernel<MODE, W32, true>), grid, dim3(256), 0, st, pd, sd);
+      else if (f32) hipLaunchKernelGGL((byte128_kernel<MODE, true, false>), grid, dim3(256), 0, st, pd, sd);
+      else hipLaunchKernelGGL((byte128_kernel<MODE, W32, false>), grid, dim3(256), 0, st, pd, sd);
+      return check_launch("byte128_kernel");
+    }
     if (pd.fast & SQ_POOL_FAST_GDN128) {
       const int ng_max = pool->group >= 32 ? 128 / pool->group : 1;
       // staging | rows | columns | q,k raw + w | misc | red | ks, qs | rc (float4), iu (float2) per (row, group)
@@ -6038,6 +6422,16 @@ int sq_pool_flags(const int32_t *bits, const int32_t *head_meta, const int32_t *
     if (w == 2) fast = fast && (group == 32 || group == 64 || group == 128);
   }
   if (fast) flags |= SQ_POOL_FAST_GDN128;
+  // byte planes on 16-byte boundaries; GDN heads of one width, 2-bit ones with at most four value groups
+  bool byte = keys == 128 && values == 128 && storage == 1 && page_bytes % 16 == 0;
+  for (int h = 0; byte && h < heads; h++) {
+    byte = byte && head_meta[4 * h] % 16 == 0;
+    if (kda) continue;
+    const int w = bits[(int64_t)h * keys];
+    for (int i = 1; i < keys; i++) byte = byte && bits[(int64_t)h * keys + i] == w;
+    if (w == 2) byte = byte && (group == 32 || group == 64 || group == 128);
+  }
+  if (byte) flags |= SQ_POOL_FAST_BYTE128;
   if (kda && keys == 128 && values == 128 && storage == 0) flags |= SQ_POOL_FAST_KDA128;
   return flags;
 }
