@@ -386,3 +386,40 @@ def test_kda_prefill_with_extreme_decays(a_log):
         for c in range(2):
             if ck_slots[b, c] > 0:
                 check_states(states[b, c], ref_states[b, c], f"state b={b} c={c}")
+
+
+@pytest.mark.parametrize("arch", ["gdn", "kda"])
+def test_prefill_order_of_sequences_changes_nothing(arch):
+    """Calls of several rounds of workgroups take the longest sequences
+    first: 66 sequences x 4 heads (more than a wave's lanes: list order), 64
+    x 5 (ranked, equal and empty ones among them) and one sequence at a time
+    give the same outputs and pages."""
+    from stepquant_amd.kernels.pool import PackedStatePool
+    print(f"case order {arch}", flush=True)
+    K, V = 128, 128
+    for B, H in ((66, 4), (64, 5)):
+        rng = np.random.default_rng(B)
+        lens = rng.integers(0, 40, B)
+        lens[:3] = (70, 0, 70)
+        cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32)
+        T = int(cu[-1])
+        plan = device_plan(make_plan(arch, np.full((H, K), 6), seed=1))
+        pools = [PackedStatePool(plan, B + 1, V) for _ in range(2)]
+        g = torch.Generator().manual_seed(9)
+        q, k, v = (torch.randn(T, H * K, generator=g).to(torch.bfloat16).to(dev()) for _ in range(3))
+        gate = (-torch.rand((T, H, K) if arch == "kda" else (T, H), generator=g)).to(dev())
+        beta = torch.rand(T, H, generator=g).to(dev())
+        slots = torch.arange(1, B + 1)
+        x = (torch.randn(B, H, K, V, generator=g) * .1).to(dev())
+        for p in pools:
+            p.encode(x, slots.to(dev()))
+        out = pools[0].extend(q, k, v, gate, beta, slots, cu, normalize=True, scale=K ** -.5)
+        for b in range(B):
+            a, e = int(cu[b]), int(cu[b + 1])
+            if a == e:
+                continue
+            one = pools[1].extend(q[a:e], k[a:e], v[a:e], gate[a:e], beta[a:e], slots[b:b + 1],
+                                  torch.tensor([0, e - a]), normalize=True, scale=K ** -.5)
+            assert torch.equal(one, out[a:e]), f"sequence {b}"
+        torch.cuda.synchronize()
+        assert torch.equal(pools[0].data, pools[1].data)
