@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 
 import torch
 
@@ -18,6 +19,9 @@ F32, BF16, F16, I32, I64 = 0, 1, 2, 3, 4
 # sq_pool.flags bits (SQ_POOL_FAST_*)
 POOL_FAST_GDN128, POOL_FAST_KDA128, POOL_FAST_BYTE128 = 1, 2, 4
 _DTYPES = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16, torch.int32: I32, torch.int64: I64}
+
+FLOATS = {t: _DTYPES[t] for t in (torch.float32, torch.bfloat16, torch.float16)}
+INTS = {t: _DTYPES[t] for t in (torch.int32, torch.int64)}
 
 _P = ctypes.c_void_p
 
@@ -154,6 +158,33 @@ def dtype_code(t: torch.Tensor) -> int:
 
 def ptr(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
+
+
+# sq_step_args as packed bytes, in the order of StepArgs' fields (all at
+# their natural offsets, no padding between them): a step's argument block
+# without a ctypes object per call
+STEP_ARGS = struct.Struct("=9Q4q6ifi")
+
+
+_step_entries = {}
+PP = ctypes.POINTER
+
+
+def step_entry(name: str):
+    """``sq_decode_step``, ``sq_decode_readout`` or ``sq_format_step`` taking the
+    pool's address and a packed STEP_ARGS block."""
+    fn = _step_entries.get(name)
+    if fn is not None:
+        return fn
+    fn = _step_entries[name] = lib()[name]  # a function object of its own: lib()'s keeps its prototype
+    fn.restype = ctypes.c_int
+    fn.argtypes = [_P, ctypes.c_char_p] + ([PP(Scratch), _P] if name == "sq_decode_readout" else [_P])
+    return fn
+
+
+def raw_stream() -> int:
+    """The current stream of the current device as a number."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def stream_handle(stream=None) -> ctypes.c_void_p:

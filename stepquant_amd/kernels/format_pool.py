@@ -10,6 +10,8 @@ in the HIP kernels behind ``sq_format_encode`` / ``sq_format_decode`` /
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from .. import _native as N
@@ -131,16 +133,24 @@ class FormatStatePool(PackedStatePool):
 
     def step(self, q, k, v, g, beta, slots, *, normalize=False, scale=1., a_log=None, dt_bias=None):
         batch = slots.numel()
-        out = torch.empty((batch, self.heads, self.values), device=self.device, dtype=q.dtype)
         if batch:
-            q, k = q.reshape(batch, -1, self.keys), k.reshape(batch, -1, self.keys)
-            v = v.reshape(batch, self.heads, self.values)
-            if self.heads % q.shape[1] or k.shape[1] != q.shape[1] or any(t.stride(-1) != 1 for t in (q, k, v)):
-                raise ValueError("invalid head layout")
-            args, keep = self._step_args(q, k, v, g, beta, slots, out, normalize, scale, a_log, dt_bias, batch,
-                                         q.shape[1])
-            N.check(N.lib().sq_format_step(self._fdesc, args, N.stream_handle()), "format step")
-        return out
+            packed = self._packed_args(q, k, v, g, beta, slots, normalize, scale, a_log, dt_bias, batch)
+            if packed is not None:
+                args, out = packed
+            else:
+                out = torch.empty((batch, self.heads, self.values), device=self.device, dtype=q.dtype)
+                q, k = q.reshape(batch, -1, self.keys), k.reshape(batch, -1, self.keys)
+                v = v.reshape(batch, self.heads, self.values)
+                if self.heads % q.shape[1] or k.shape[1] != q.shape[1] or any(t.stride(-1) != 1 for t in (q, k, v)):
+                    raise ValueError("invalid head layout")
+                args, keep = self._step_args(q, k, v, g, beta, slots, out, normalize, scale, a_log, dt_bias, batch,
+                                             q.shape[1])
+                args = bytes(args)
+            rc = N.step_entry("sq_format_step")(ctypes.addressof(self._fdesc), args, N.raw_stream())
+            if rc:
+                N.check(rc, "format step")
+            return out
+        return torch.empty((batch, self.heads, self.values), device=self.device, dtype=q.dtype)
 
     def extend(self, *args, **kwargs):
         raise ValueError("chunked prefill writes STEPQuant pages; baseline formats use decode/encode")

@@ -310,6 +310,43 @@ class PackedStatePool:
         keep = (q, k, v, g, beta, a_log, dt_bias, idx)
         return args, keep
 
+    def _packed_args(self, q, k, v, g, beta, slots, normalize, scale, a_log, dt_bias, batch):
+        """(packed argument block, output) of a step whose tensors the kernels
+        take as they are: 2-D q, k, v rows, contiguous gates of one type and a
+        slot vector on the pool's device.  None for any other call, which
+        ``_step_args`` converts or refuses; a step's launch costs less than
+        its host work, so the usual call skips the views and conversions."""
+        dt = q.dtype
+        code = N.FLOATS.get(dt)
+        gdt = N.FLOATS.get(g.dtype)
+        slot_code = N.INTS.get(slots.dtype)
+        if code is None or gdt is None or slot_code is None or k.dtype != dt or v.dtype != dt \
+                or beta.dtype != g.dtype or q.dim() != 2 or k.dim() != 2 or v.dim() != 2 or slots.dim() != 1:
+            return None
+        K, H, V, dev = self.keys, self.heads, self.values, self.device
+        (rows, width), (qs, q1), (ks, k1), (vs, v1) = q.shape, q.stride(), k.stride(), v.stride()
+        hq = width // K
+        per = H * K if self.plan.architecture == "kda" else H
+        if q1 != 1 or k1 != 1 or v1 != 1 or rows != batch or hq * K != width or not hq or H % hq \
+                or k.shape != q.shape or v.shape != (batch, H * V) or g.numel() != batch * per \
+                or beta.numel() != batch * H or not (g.is_contiguous() and beta.is_contiguous()
+                                                     and slots.is_contiguous()) \
+                or g.device != dev or beta.device != dev or slots.device != dev or q.device != dev \
+                or k.device != dev or v.device != dev:
+            return None
+        a_ptr = d_ptr = 0
+        if a_log is not None or dt_bias is not None:
+            if a_log is None or dt_bias is None or a_log.dtype != g.dtype or dt_bias.dtype != g.dtype or a_log.numel() != H \
+                    or dt_bias.numel() != per or not (a_log.is_contiguous() and dt_bias.is_contiguous()) \
+                    or a_log.device != dev or dt_bias.device != dev:
+                return None
+            a_ptr, d_ptr = a_log.data_ptr(), dt_bias.data_ptr()
+        out = torch.empty((batch, H, V), device=dev, dtype=dt)
+        return N.STEP_ARGS.pack(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr(), a_ptr, d_ptr, out.data_ptr(),
+            slots.data_ptr(), batch, qs, ks, vs, hq, code, gdt, code, slot_code, bool(normalize),
+            ctypes.c_float(scale).value, 0), out
+
     def step(self, q, k, v, g, beta, slots, *, normalize=False, scale=1., a_log=None, dt_bias=None):
         self.wait()
         if self.deferred is not None and not self.deferred.attention_windows:
@@ -317,24 +354,32 @@ class PackedStatePool:
         batch = slots.numel()
         if not batch:
             return torch.empty((0, self.heads, self.values), device=q.device, dtype=q.dtype)
-        q = q.reshape(batch, -1, self.keys)
-        k = k.reshape(batch, -1, self.keys)
-        v = v.reshape(batch, self.heads, self.values)
-        if q.stride(-1) != 1 or k.stride(-1) != 1 or v.stride(-1) != 1:
-            raise ValueError("head coordinates must be contiguous")
-        hq = q.shape[1]
-        if self.heads % hq or k.shape[1] != hq:
-            raise ValueError("value heads must be divisible by query heads")
-        out = torch.empty((batch, self.heads, self.values), device=q.device, dtype=q.dtype)
-        args, keep = self._step_args(q, k, v, g, beta, slots, out, normalize, scale, a_log, dt_bias, batch, hq)
+        packed = self._packed_args(q, k, v, g, beta, slots, normalize, scale, a_log, dt_bias, batch)
+        if packed is None:
+            q = q.reshape(batch, -1, self.keys)
+            k = k.reshape(batch, -1, self.keys)
+            v = v.reshape(batch, self.heads, self.values)
+            if q.stride(-1) != 1 or k.stride(-1) != 1 or v.stride(-1) != 1:
+                raise ValueError("head coordinates must be contiguous")
+            hq = q.shape[1]
+            if self.heads % hq or k.shape[1] != hq:
+                raise ValueError("value heads must be divisible by query heads")
+            out = torch.empty((batch, self.heads, self.values), device=q.device, dtype=q.dtype)
+            args, keep = self._step_args(q, k, v, g, beta, slots, out, normalize, scale, a_log, dt_bias, batch, hq)
+            args = bytes(args)
+        else:
+            args, out = packed
         if self.writeback_stream is None:
-            N.check(N.lib().sq_decode_step(self._desc, args, N.stream_handle()), "decode step")
+            rc = N.step_entry("sq_decode_step")(ctypes.addressof(self._desc), args, N.raw_stream())
+            if rc:
+                N.check(rc, "decode step")
             return out
         if batch > self.scratch[0].shape[0]:
             raise ValueError("active batch exceeds the state pool workspace capacity")
         update_key, decay, delta, partial, stable_slots = (t[:batch] for t in self.scratch)
         scratch = self._scratch_desc(update_key, decay, delta, stable_slots)
-        N.check(N.lib().sq_decode_readout(self._desc, args, scratch, N.stream_handle()), "decode readout")
+        N.check(N.step_entry("sq_decode_readout")(ctypes.addressof(self._desc), args, scratch, N.raw_stream()),
+                "decode readout")
         self._schedule_writeback(update_key, decay, delta, partial, stable_slots)
         return out
 
@@ -379,11 +424,13 @@ class PackedStatePool:
             # offsets known on the host: checked here, copied without a wait
             cu_host = offsets = torch.as_tensor(cu_seqlens).to(torch.int32).reshape(-1).contiguous()
             cu = None  # copied below, with the checkpoints when they are host tensors too
+        # (numpy below: host work here is on the step's critical path)
+        cu_n = offsets.numpy()
         total = 0
-        if offsets.numel() > 1:
-            total = int(offsets[-1])
-            _check_offsets(int(offsets[0]), int((offsets[1:] < offsets[:-1]).sum()))
-        batch = offsets.numel() - 1
+        if cu_n.size > 1:
+            total = int(cu_n[-1])
+            _check_offsets(int(cu_n[0]), int((cu_n[1:] < cu_n[:-1]).sum()))
+        batch = cu_n.size - 1
         if batch < 0:
             raise ValueError("cu_seqlens needs at least one entry")
         slots_t = _indices(slots, dev)
@@ -426,23 +473,21 @@ class PackedStatePool:
             cs_h = torch.as_tensor(checkpoint_slots).to(torch.int64).reshape(batch, -1)
             if cs_h.shape != ck_h.shape:
                 raise ValueError("one slot per checkpoint")
-            lengths_h = (cu_host[1:] - cu_host[:-1]).reshape(batch, 1)
-            used = (ck_h > 0) & (ck_h <= lengths_h)
             # used positions must not decrease along a row: each one is at
-            # least the largest used position before it (numpy: host work
-            # here is on the step's critical path)
-            ck_n, used_n = ck_h.numpy(), used.numpy()
+            # least the largest used position before it
+            ck_n, cs_n = ck_h.numpy(), cs_h.numpy()
+            used_n = (ck_n > 0) & (ck_n <= (cu_n[1:] - cu_n[:-1])[:, None])
             seen = np.maximum.accumulate(np.where(used_n, ck_n, 0), axis=1)
             if (used_n[:, 1:] & (ck_n[:, 1:] < seen[:, :-1])).any():
                 raise ValueError("checkpoints of a sequence must be ascending")
-            cs_h = torch.where(used, cs_h, torch.zeros_like(cs_h))
             # offsets, checkpoints and their slots in one pinned buffer: one copy
-            n_cs, n_ck, n_cu = cs_h.numel(), ck_h.numel(), cu_host.numel()
+            n_cs, n_ck, n_cu = cs_n.size, ck_n.size, cu_n.size
             packed = torch.empty(n_cs + (n_ck + n_cu + 1) // 2, dtype=torch.int64, pin_memory=True)
-            packed[:n_cs] = cs_h.reshape(-1)
-            p32 = packed[n_cs:].view(torch.int32)
-            p32[:n_cu] = cu_host
-            p32[n_cu:n_cu + n_ck] = ck_h.reshape(-1)
+            packed_n = packed.numpy()
+            np.multiply(cs_n, used_n, out=packed_n[:n_cs].reshape(cs_n.shape))  # unused positions: slot 0
+            p32 = packed_n[n_cs:].view(np.int32)
+            p32[:n_cu] = cu_n
+            p32[n_cu:n_cu + n_ck] = ck_n.reshape(-1)
             packed = packed.to(dev, non_blocking=True)
             ck_slots = packed[:n_cs].view(cs_h.shape)
             d32 = packed[n_cs:].view(torch.int32)
