@@ -5995,14 +5995,17 @@ __global__ __launch_bounds__(256) void format_kernel(FmtDev F, StepDev S) {
 
 // =====================================================================
 // The fused step on SYMMETRIC pages with K = V = 128 (one group per row) and
-// the head's code rows contiguous: format_kernel's operations in its order
-// for one code width W, so both give the same bytes.  The codes are staged by
+// on FP32 pages (W = 32: no codes, the values stay in registers), the head's
+// rows contiguous: format_kernel's operations in its order for one code width
+// W, so both give the same bytes.  The codes are staged by
 // direct global-to-LDS loads issued with every other input; row maxima
 // (order-free) are reduced between lanes; a row's scale, its reciprocal and
 // its retention are formed once, not by each of its 32 lanes; codes are
 // rounded by the addition of 1.5 2^23 and packed W bits wide without
-// branches.  Four workgroups per CU (128 registers).  Bound by VALU issue.
-// sym_int6, B = 256, 32 heads: 97 us a step, 219 us in format_kernel.
+// branches.  Four workgroups per CU (128 registers).  sym_int6, B = 256, 32
+// heads: 97 us a step, 219 us in format_kernel; bound by VALU issue.  FP32
+// pages of that size: 227 us, 290 us in format_kernel; bound by memory (1.07
+// GB read and written a step, 4.7 TB/s; a large copy reaches 4.9).
 // =====================================================================
 namespace sym {
 
@@ -6023,8 +6026,9 @@ template <int W, bool QW4>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void sym128_step_kernel(FmtDev F,
                                                                                                    StepDev S) {
 #pragma clang fp contract(off)
+  constexpr bool CODES = W < 32;                    // W == 32: an FP32 page, its values go through registers only
   constexpr int ROW = FV * W / 8, CODE = FK * ROW;  // bytes of a row's and a head's codes
-  __shared__ __align__(16) uint8_t stg[CODE + 32];
+  __shared__ __align__(16) uint8_t stg[CODES ? CODE + 32 : 16];
   __shared__ float2 kq[FK], sz[FK], si[FK];  // k, q | old scale and zero point | new scale and its reciprocal
   __shared__ float ret[FK], red[4 * FK];
   const int H = F.H, h = blockIdx.x, b = blockIdx.y;
@@ -6040,7 +6044,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
   uint8_t *code = page + ld_uniform(F.offsets + hr);
   const int shift = (int)((uintptr_t)code & 15);
   // ---- every load of the tile, then the first use
-  if (shift == 0) {
+  float x[16][4];
+  if constexpr (!CODES) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) __builtin_memcpy(x[r], code + (rg + 8 * r) * ROW + 4 * j0, 16);
+  } else if (shift == 0) {
 #pragma unroll
     for (int k = 0; k < CODE / 4096; k++)
       __builtin_amdgcn_global_load_lds((fast::gptr_t)((const uint4 *)code + tid + 256 * k),
@@ -6048,7 +6056,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
   } else {
     stage_in(code, CODE, stg, tid, 256);
   }
-  const int rpos = F.rows[hr + i];
+  const int rpos = CODES ? F.rows[hr + i] : 0;
   const int hk = (h * S.hk_mul) >> 20;
   const int64_t qb = (int64_t)b * S.q_stride + (int64_t)hk * FK, kb = (int64_t)b * S.k_stride + (int64_t)hk * FK;
   const int64_t gi = F.kda ? bh * FK + i : bh, di = F.kda ? hr + i : h;
@@ -6065,7 +6073,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
     alog = __expf(load_val(S.a_log, S.gate_dtype, h));
     bt = 1.0f / (1.0f + __expf(-bt));
   }
-  const float os = h2f(page_half(page, rpos)), oz = h2f(page_half(page, rpos + 2));
+  const float os = CODES ? h2f(page_half(page, rpos)) : 0.0f, oz = CODES ? h2f(page_half(page, rpos + 2)) : 0.0f;
   const float sq = fast::wave_sum(q2[0] * q2[0] + q2[1] * q2[1]), sk = fast::wave_sum(k2[0] * k2[0] + k2[1] * k2[1]);
   const float nq = S.normalize ? 1.0f / __builtin_sqrtf(sq + 1e-6f) : 1.0f;
   const float nk = S.normalize ? 1.0f / __builtin_sqrtf(sk + 1e-6f) : 1.0f;
@@ -6083,22 +6091,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
   __syncthreads();
 
   // ---- x = ((code - z) s) d, k^T x
-  float x[16][4];
   float kr[4] = {0.f, 0.f, 0.f, 0.f};
   const bool aligned = (shift & 3) == 0;
   const int pos0 = shift + rg * ROW + j0 * W / 8;  // rows rg + 8 r are 8 ROW bytes apart
 #pragma unroll
   for (int r = 0; r < 16; r++) {
     const int row = rg + 8 * r, pos = pos0 + r * 8 * ROW;
-    uint32_t word;
-    if (W == 8 && aligned) word = *(const uint32_t *)(stg + pos);
+    uint32_t word = 0;
+    if (!CODES) word = 0;
+    else if (W == 8 && aligned) word = *(const uint32_t *)(stg + pos);
     else if (W == 4 && aligned) word = *(const uint16_t *)(stg + pos);
     else word = lds_word(stg, pos);
     const float2 o = sz[row];
     const float d = ret[row], k = kq[row].x;
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-      x[r][c] = (((float)((word >> (c * W)) & ((1u << W) - 1u)) - o.y) * o.x) * d;
+      if constexpr (CODES) x[r][c] = ((float)((word >> (c * W)) & ((1u << W) - 1u)) - o.y) * o.x;
+      x[r][c] = x[r][c] * d;
       kr[c] = kr[c] + k * x[r][c];
     }
   }
@@ -6130,6 +6139,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
 #pragma unroll
   for (int c = 0; c < 4; c++) o[c] = fast::rg8_sum(o[c]);
   if (rg == 0) store4(S.out, S.out_dtype, bh * FV + j0, o);
+  if constexpr (!CODES) {
+    uint32_t at = rg * ROW + 4 * j0;
+    asm volatile("" : "+v"(at));  // addresses made anew: kept from the loads on, they cost 10 spills
+#pragma unroll
+    for (int r = 0; r < 16; r++) __builtin_memcpy(code + (at + 8 * ROW * r), x[r], 16);
+    return;
+  }
   float amax = 0.0f;
 #pragma unroll
   for (int r = 0; r < 16; r++) amax = fmaxf(amax, rowm[r]);
@@ -6154,7 +6170,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
     red[wave * FK + rg + 8 * (8 * b5 + 4 * b4 + 2 * b3 + r)] = fmaxf(keep, fast::dpp<0x128>(send));  // row_ror:8
   }
   __syncthreads();
-  constexpr float Lf = (float)((1 << (W - 1)) - 1);
+  constexpr int WC = CODES ? W : 8;
+  constexpr float Lf = (float)((1 << (WC - 1)) - 1);
   if (tid < FK) {
     const float m = fmaxf(fmaxf(fmaxf(fmaxf(0.0f, red[i]), red[FK + i]), red[2 * FK + i]), red[3 * FK + i]);
     uint32_t hb;
@@ -6180,7 +6197,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
         const float y = decltype(ieee)::value ? x[r][c] / u.x : div_half(x[r][c], u.x, u.y);
         t[c] = __builtin_amdgcn_fmed3f(y + MAGIC, MAGIC - Lf, MAGIC + Lf) + Lf;
       }
-      const uint32_t word = pack<W>(t);
+      const uint32_t word = pack<WC>(t);
       const int pos = pos0 + r * 8 * ROW;
       if (W == 8 && aligned) *(uint32_t *)(stg + pos) = word;
       else if (W == 4 && aligned) *(uint16_t *)(stg + pos) = (uint16_t)word;
@@ -7078,9 +7095,11 @@ int sq_format_step(const sq_format_pool *pool, const sq_step_args *args, void *s
   FmtDev fd = to_fmt(pool);
   fd.slots = args->slots;
   fd.slots_dtype = args->slots_dtype;
-  // fd.stage: code rows contiguous; heads and batch as the K = V = 128 packed kernels (grid, key-head factor)
-  if (pool->kind == SQ_FMT_SYMMETRIC && pool->keys == 128 && pool->values == 128 && fd.stage > 0 &&
-      pool->heads <= 1024 && args->batch > 0 && args->batch <= 65535) {
+  // contiguous rows (fd.stage for codes); heads and batch as the K = V = 128 packed kernels (grid, key-head factor)
+  const bool codes = pool->kind == SQ_FMT_SYMMETRIC && fd.stage > 0;
+  const bool fp32 = pool->kind == SQ_FMT_FP32 && (pool->flags & SQ_FMT_ROWS_CONTIGUOUS);
+  if ((codes || fp32) && pool->keys == 128 && pool->values == 128 && pool->heads <= 1024 && args->batch > 0 &&
+      args->batch <= 65535) {
     const int ratio = pool->heads / sd.HK;
     sd.hk_mul = ((1 << 20) + ratio - 1) / ratio;
     const dim3 grid((unsigned)pool->heads, (unsigned)args->batch);
@@ -7088,6 +7107,7 @@ int sq_format_step(const sq_format_pool *pool, const sq_step_args *args, void *s
       hipLaunchKernelGGL(sd.qkv_dtype == SQ_F32 ? f32 : other, grid, dim3(256), 0, (hipStream_t)stream, fd, sd);
       return check_launch("sym128_step_kernel");
     };
+    if (fp32) return go(sym::sym128_step_kernel<32, true>, sym::sym128_step_kernel<32, false>);
     if (pool->bits == 4) return go(sym::sym128_step_kernel<4, true>, sym::sym128_step_kernel<4, false>);
     if (pool->bits == 6) return go(sym::sym128_step_kernel<6, true>, sym::sym128_step_kernel<6, false>);
     return go(sym::sym128_step_kernel<8, true>, sym::sym128_step_kernel<8, false>);
