@@ -5994,9 +5994,9 @@ __global__ __launch_bounds__(256) void format_kernel(FmtDev F, StepDev S) {
 }
 
 // =====================================================================
-// The fused step on SYMMETRIC pages with K = V = 128 (one group per row) and
-// on FP32 pages (W = 32: no codes, the values stay in registers), the head's
-// rows contiguous: format_kernel's operations in its order for one code width
+// The fused step on SYMMETRIC (one group per row), dual-axis (DSQ) and FP32
+// pages (W = 32: no codes, the values stay in registers) with K = V = 128, the
+// head's rows contiguous: format_kernel's operations in its order for one code width
 // W, so both give the same bytes.  The codes are staged by
 // direct global-to-LDS loads issued with every other input; row maxima
 // (order-free) are reduced between lanes; a row's scale, its reciprocal and
@@ -6006,12 +6006,21 @@ __global__ __launch_bounds__(256) void format_kernel(FmtDev F, StepDev S) {
 // heads: 97 us a step, 219 us in format_kernel; bound by VALU issue.  FP32
 // pages of that size: 227 us, 290 us in format_kernel; bound by memory (1.07
 // GB read and written a step, 4.7 TB/s; a large copy reaches 4.9).
+// DSQ: the row means need each row's columns in a fixed order, so |x| passes
+// through LDS half the rows at a time, in the place of the codes, and 8
+// threads sum a row; 155 registers, three workgroups per CU (held to 128 it
+// spilled 37 values: 304 us).  dsq_int6, that size: 174 us, 430 us in
+// format_kernel; bound by VALU issue (two quotients a value).
 // =====================================================================
 namespace sym {
 
 constexpr int FK = 128, FV = 128;
 
 // four codes from 1.5 2^23 + code, column c at bits [c W, c W + W)
+template <int N>
+struct Width {
+  static constexpr int value = N;
+};
 template <int W>
 __device__ __forceinline__ uint32_t pack(const float t[4]) {
   const uint32_t a = __float_as_uint(t[0]), b = __float_as_uint(t[1]), c = __float_as_uint(t[2]),
@@ -6022,13 +6031,14 @@ __device__ __forceinline__ uint32_t pack(const float t[4]) {
   return W == 4 ? (x & 0xffu) | ((x >> 8) & 0xff00u) : (x & 0xfffu) | ((x >> 4) & 0xfff000u);
 }
 
-template <int W, bool QW4>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void sym128_step_kernel(FmtDev F,
+template <int W, bool DSQ, bool QW4>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DSQ ? 3 : 4))) void sym128_step_kernel(FmtDev F,
                                                                                                    StepDev S) {
 #pragma clang fp contract(off)
   constexpr bool CODES = W < 32;                    // W == 32: an FP32 page, its values go through registers only
   constexpr int ROW = FV * W / 8, CODE = FK * ROW;  // bytes of a row's and a head's codes
-  __shared__ __align__(16) uint8_t stg[CODES ? CODE + 32 : 16];
+  constexpr int PITCH = FV + 4;                     // DSQ: |x| of half the rows takes the place of the codes
+  __shared__ __align__(16) uint8_t stg[DSQ ? FK / 2 * PITCH * 4 : CODES ? CODE + 32 : 16];
   __shared__ float2 kq[FK], sz[FK], si[FK];  // k, q | old scale and zero point | new scale and its reciprocal
   __shared__ float ret[FK], red[4 * FK];
   const int H = F.H, h = blockIdx.x, b = blockIdx.y;
@@ -6073,7 +6083,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
     alog = __expf(load_val(S.a_log, S.gate_dtype, h));
     bt = 1.0f / (1.0f + __expf(-bt));
   }
-  const float os = CODES ? h2f(page_half(page, rpos)) : 0.0f, oz = CODES ? h2f(page_half(page, rpos + 2)) : 0.0f;
+  const float os = CODES ? h2f(page_half(page, rpos)) : 0.0f;
+  const float oz = CODES && !DSQ ? h2f(page_half(page, rpos + 2)) : 0.0f;
+  float cj[4];
+  const int cpos = DSQ ? F.columns[h] + 4 * j0 : 0;
+#pragma unroll
+  for (int c = 0; c < 4; c++) cj[c] = DSQ ? h2f(page_half(page, cpos + 4 * c)) : 0.0f;
   const float sq = fast::wave_sum(q2[0] * q2[0] + q2[1] * q2[1]), sk = fast::wave_sum(k2[0] * k2[0] + k2[1] * k2[1]);
   const float nq = S.normalize ? 1.0f / __builtin_sqrtf(sq + 1e-6f) : 1.0f;
   const float nk = S.normalize ? 1.0f / __builtin_sqrtf(sk + 1e-6f) : 1.0f;
@@ -6106,7 +6121,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
     const float d = ret[row], k = kq[row].x;
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-      if constexpr (CODES) x[r][c] = ((float)((word >> (c * W)) & ((1u << W) - 1u)) - o.y) * o.x;
+      const uint32_t u = (word >> (CODES ? c * W : 0)) & ((1u << (W & 31)) - 1u);
+      if constexpr (DSQ) x[r][c] = (o.x * cj[c]) * (float)((int)u - ((1 << (W - 1)) - 1));
+      else if constexpr (CODES) x[r][c] = ((float)u - o.y) * o.x;
       x[r][c] = x[r][c] * d;
       kr[c] = kr[c] + k * x[r][c];
     }
@@ -6149,6 +6166,112 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
   float amax = 0.0f;
 #pragma unroll
   for (int r = 0; r < 16; r++) amax = fmaxf(amax, rowm[r]);
+  constexpr int WC = CODES ? W : 8;
+  constexpr float Lf = (float)((1 << (WC - 1)) - 1);
+  constexpr float MAGIC = 12582912.0f;  // 1.5 2^23: adding it rounds to an integer in the low bits
+  auto put_codes = [&](int r, const float t[4]) {
+    const uint32_t word = pack<WC>(t);
+    const int pos = pos0 + r * 8 * ROW;
+    if (W == 8 && aligned) *(uint32_t *)(stg + pos) = word;
+    else if (W == 4 && aligned) *(uint16_t *)(stg + pos) = (uint16_t)word;
+    else lds_put_bytes(stg, pos, word, W / 2);
+  };
+  auto write_codes = [&]() {
+    __syncthreads();
+    if (shift == 0) {
+#pragma unroll
+      for (int k = 0; k < CODE / 4096; k++) ((uint4 *)code)[tid + 256 * k] = ((const uint4 *)stg)[tid + 256 * k];
+    } else {
+      stage_out(code, CODE, stg, tid, 256);
+    }
+  };
+  if constexpr (DSQ) {
+    // ---- row means of |x| in format_kernel's order: column 32 a + 8 n + l is
+    // term a of accumulator n of lane l; 8 threads per row, thread l
+    float *xs = (float *)stg;
+    const int wr = 16 * wave + 2 * (l >> 3), lane = l & 7;  // rows 2 apart in a wave: distinct banks
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < 8; r++) {
+        const float *v = x[8 * p + r];
+        *(float4 *)(xs + (rg + 8 * r) * PITCH + j0) = make_float4(fabsf(v[0]), fabsf(v[1]), fabsf(v[2]), fabsf(v[3]));
+      }
+      __syncthreads();
+#pragma unroll 1
+      for (int u = 0; u < 2; u++) {
+        const float *row = xs + (wr + u) * PITCH + lane;
+        float acc[4];
+#pragma unroll
+        for (int n = 0; n < 4; n++) acc[n] = ((row[8 * n] + row[32 + 8 * n]) + row[64 + 8 * n]) + row[96 + 8 * n];
+        const float sl = ((acc[0] + acc[1]) + acc[2]) + acc[3];
+        float total = sl;
+        total += row_shl<1>(sl);
+        total += row_shl<2>(sl);
+        total += row_shl<3>(sl);
+        total += row_shl<4>(sl);
+        total += row_shl<5>(sl);
+        total += row_shl<6>(sl);
+        total += row_shl<7>(sl);
+        if (lane == 0) red[64 * p + wr + u] = total;
+      }
+    }
+    __syncthreads();
+    if (tid < FK) {
+      float m = red[i] / (float)FV;
+      m = m < 1e-20f ? 1e-20f : m;
+      uint32_t hb;
+      const float s = fp16_scale(__builtin_sqrtf(m), &hb);
+      si[i] = make_float2(s, 1.0f / s);
+      put_page_half(page, rpos, hb);
+    }
+    __syncthreads();
+    settle();
+    // ---- y = x / r, column maxima, codes of y / c.  Both quotients from
+    // reciprocals with one correction where that is exact for every value of
+    // the wave (scales lie in [2^-24, 2^16): |y| in [2^-76, 2^84] and its
+    // quotients below 2^108 and above 2^-92), else by IEEE division
+    auto finish = [&](auto ieee) {
+      float mx[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const float2 u = si[rg + 8 * r];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          x[r][c] = decltype(ieee)::value ? x[r][c] / u.x : div_half(x[r][c], u.x, u.y);
+          mx[c] = fmaxf(mx[c], fabsf(x[r][c]));
+        }
+      }
+      settle();
+      float2 v[4];
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        uint32_t hb;
+        const float s = fp16_scale(fast::rg8_max_nonneg(mx[c]) / Lf, &hb);
+        v[c] = make_float2(s, 1.0f / s);
+        if (rg == 0) {
+          put_page_half(page, cpos + 4 * c, hb);
+          put_page_half(page, cpos + 4 * c + 2, 0u);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        float t[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          const float y = decltype(ieee)::value ? x[r][c] / v[c].x : div_half(x[r][c], v[c].x, v[c].y);
+          t[c] = __builtin_amdgcn_fmed3f(y + MAGIC, MAGIC - Lf, MAGIC + Lf) + Lf;
+        }
+        put_codes(r, t);
+      }
+    };
+    // one form for the whole wave: the column maxima are taken across its lanes
+    if (__all(amin >= 0x1p-60f && amax <= 0x1p+60f)) finish(BoolTag<false>());
+    else finish(BoolTag<true>());
+    write_codes();
+    return;
+  }
   // maxima over the wave's 8 column groups (lane bits 3, 4, 5), scattered: a lane ends with two rows
   const int b3 = (tid >> 3) & 1, b4 = (tid >> 4) & 1, b5 = (tid >> 5) & 1;
   float p8[8], p4[4];
@@ -6170,8 +6293,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
     red[wave * FK + rg + 8 * (8 * b5 + 4 * b4 + 2 * b3 + r)] = fmaxf(keep, fast::dpp<0x128>(send));  // row_ror:8
   }
   __syncthreads();
-  constexpr int WC = CODES ? W : 8;
-  constexpr float Lf = (float)((1 << (WC - 1)) - 1);
   if (tid < FK) {
     const float m = fmaxf(fmaxf(fmaxf(fmaxf(0.0f, red[i]), red[FK + i]), red[2 * FK + i]), red[3 * FK + i]);
     uint32_t hb;
@@ -6186,7 +6307,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
   // reciprocal with one correction where that is exact for every value of
   // the thread (scales are at least 2^-24, so 2^101 bounds the quotients),
   // else by IEEE division
-  constexpr float MAGIC = 12582912.0f;  // 1.5 2^23: adding it rounds to an integer in the low bits
   auto codes = [&](auto ieee) {
 #pragma unroll
     for (int r = 0; r < 16; r++) {
@@ -6197,22 +6317,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void s
         const float y = decltype(ieee)::value ? x[r][c] / u.x : div_half(x[r][c], u.x, u.y);
         t[c] = __builtin_amdgcn_fmed3f(y + MAGIC, MAGIC - Lf, MAGIC + Lf) + Lf;
       }
-      const uint32_t word = pack<WC>(t);
-      const int pos = pos0 + r * 8 * ROW;
-      if (W == 8 && aligned) *(uint32_t *)(stg + pos) = word;
-      else if (W == 4 && aligned) *(uint16_t *)(stg + pos) = (uint16_t)word;
-      else lds_put_bytes(stg, pos, word, W / 2);
+      put_codes(r, t);
     }
   };
   if (amin >= 0x1p-100f && amax <= 0x1p+101f) codes(BoolTag<false>());
   else codes(BoolTag<true>());
-  __syncthreads();
-  if (shift == 0) {
-#pragma unroll
-    for (int k = 0; k < CODE / 4096; k++) ((uint4 *)code)[tid + 256 * k] = ((const uint4 *)stg)[tid + 256 * k];
-  } else {
-    stage_out(code, CODE, stg, tid, 256);
-  }
+  write_codes();
 }
 
 }  // namespace sym
@@ -7096,7 +7206,7 @@ int sq_format_step(const sq_format_pool *pool, const sq_step_args *args, void *s
   fd.slots = args->slots;
   fd.slots_dtype = args->slots_dtype;
   // contiguous rows (fd.stage for codes); heads and batch as the K = V = 128 packed kernels (grid, key-head factor)
-  const bool codes = pool->kind == SQ_FMT_SYMMETRIC && fd.stage > 0;
+  const bool dsq = pool->kind == SQ_FMT_DSQ, codes = fd.stage > 0;
   const bool fp32 = pool->kind == SQ_FMT_FP32 && (pool->flags & SQ_FMT_ROWS_CONTIGUOUS);
   if ((codes || fp32) && pool->keys == 128 && pool->values == 128 && pool->heads <= 1024 && args->batch > 0 &&
       args->batch <= 65535) {
@@ -7107,10 +7217,15 @@ int sq_format_step(const sq_format_pool *pool, const sq_step_args *args, void *s
       hipLaunchKernelGGL(sd.qkv_dtype == SQ_F32 ? f32 : other, grid, dim3(256), 0, (hipStream_t)stream, fd, sd);
       return check_launch("sym128_step_kernel");
     };
-    if (fp32) return go(sym::sym128_step_kernel<32, true>, sym::sym128_step_kernel<32, false>);
-    if (pool->bits == 4) return go(sym::sym128_step_kernel<4, true>, sym::sym128_step_kernel<4, false>);
-    if (pool->bits == 6) return go(sym::sym128_step_kernel<6, true>, sym::sym128_step_kernel<6, false>);
-    return go(sym::sym128_step_kernel<8, true>, sym::sym128_step_kernel<8, false>);
+    if (fp32) return go(sym::sym128_step_kernel<32, false, true>, sym::sym128_step_kernel<32, false, false>);
+    auto width = [&](auto w) {
+      constexpr int W = decltype(w)::value;
+      return dsq ? go(sym::sym128_step_kernel<W, true, true>, sym::sym128_step_kernel<W, true, false>)
+                 : go(sym::sym128_step_kernel<W, false, true>, sym::sym128_step_kernel<W, false, false>);
+    };
+    if (pool->bits == 4) return width(sym::Width<4>());
+    if (pool->bits == 6) return width(sym::Width<6>());
+    return width(sym::Width<8>());
   }
   return launch_format<FMT_STEP>(pool, fd, sd, args->batch, (hipStream_t)stream);
 }

@@ -1,4 +1,4 @@
-"""Symmetric and fp32 format steps at K = V = 128: the width-compiled kernel against the
+"""Symmetric, dual-axis and fp32 format steps at K = V = 128: the width-compiled kernel against the
 general one (MI355X), the same operations in the same order, so outputs and
 pages agree bit for bit; zeros, infinities and NaN, scales at both ends of
 fp16, and pages on odd offsets among them."""
@@ -14,19 +14,26 @@ pytestmark = pytest.mark.gpu
     (4, "gdn", torch.bfloat16, torch.float32, 0), (6, "gdn", torch.float32, torch.bfloat16, 0),
     (8, "kda", torch.float16, torch.float32, 0), (6, "kda", torch.bfloat16, torch.float16, 4),
     (32, "gdn", torch.bfloat16, torch.float32, 0), (32, "kda", torch.float32, torch.bfloat16, 4),
+    ("dsq4", "gdn", torch.bfloat16, torch.float32, 0), ("dsq6", "kda", torch.float32, torch.bfloat16, 0),
+    ("dsq6", "gdn", torch.float16, torch.float32, 4), ("dsq8", "gdn", torch.bfloat16, torch.float32, 2),
     (4, "gdn", torch.bfloat16, torch.float32, 2), (8, "gdn", torch.float32, torch.float32, 6)])
 def test_sym_kernel_matches_the_general_one(bits, arch, dtype, gate, pad):
     """FP32 pages among them (32 bits).  ``pad`` bytes before the first code row move every region off its alignment."""
-    from stepquant_amd.formats import FormatPlan, get_format
+    from stepquant_amd.formats import FormatPlan, StateFormat, get_format
     from stepquant_amd.kernels.format_pool import FormatStatePool, format_layout
     print(f"case {bits} {arch} {dtype} pad={pad}", flush=True)
     H, K, V, B = 3, 128, 128, 4
     HK = 3 if arch == "kda" else 1
-    spec = get_format(f"sym_int{bits}_g128" if bits < 32 else "fp32")
+    name, bits = str(bits), int(str(bits)[-2:].strip("q"))
+    if "dsq" in name:
+        spec = StateFormat(f"dsq_int{bits}", "dsq", bits, 128, "k")
+    else:
+        spec = get_format(f"sym_int{bits}_g128" if bits < 32 else "fp32")
     plan = FormatPlan(arch, torch.full((H, K), bits).to(dev()), torch.ones(H, K, device=dev()))
     offsets, rows, columns, size = format_layout(plan, V, spec)
     if pad:
-        offsets, rows, size = [o + pad for o in offsets], [r + 4 * pad for r in rows], size + 4 * pad
+        offsets, rows, size = [o + pad for o in offsets], [r + 4 * pad for r in rows], size + 8 * pad
+        columns = [c + 8 * pad for c in columns]
     pools = [FormatStatePool(plan, B + 1, V, spec, layout=(offsets, rows, columns, size)) for _ in range(2)]
     assert pools[0]._fdesc.flags
     pools[1]._fdesc.flags = 0  # rows read from the page by the general kernel
