@@ -4752,11 +4752,11 @@ constexpr int OFF_QB = OFF_KB + 2 * C * RP * 2;   // bf16 2 x [C][RP] q e^{G - G
 constexpr int OFF_A = OFF_QB + 2 * C * RP * 2;   // f32 [C][AP] A (zero on and above the diagonal)
 constexpr int OFF_M = OFF_A + C * AP * 4;         // bf16 2 x [16][PP] -A10 (hi, lo): rows 16.., columns 0..15
 constexpr int OFF_PM = OFF_M + 2 * 16 * PP * 2;   // bf16 2 x [C][PP] P (hi, lo), zero above the diagonal
-constexpr int OFF_SM = OFF_PM + 2 * C * PP * 2;   // f32 [4][C] beta, nk, nq; flags
-constexpr int OFF_EC = OFF_SM + 4 * C * 4;        // f32 [KV] e^{G_C}
+constexpr int OFF_SM = OFF_PM + 2 * C * PP * 2;   // f32 [5][C] beta (by chunk parity), nk, nq; flags
+constexpr int OFF_EC = OFF_SM + 5 * C * 4;        // f32 [KV] e^{G_C}
 constexpr int LDS_BYTES = OFF_EC + KV * 4;
 static_assert(LDS_BYTES <= 160 * 1024, "LDS of the KDA chunk kernel");
-enum { SM_BETA = 0, SM_NK, SM_NQ, SM_FLAG };
+enum { SM_BETA = 0, SM_NK = 2, SM_NQ, SM_FLAG };  // beta: rows 0 and 1, the chunk's parity
 // a chunk whose decay exceeds 2^GROW_MAX on some channel takes the pairwise path
 constexpr float GROW_MAX = 96.0f;
 
@@ -5016,8 +5016,9 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
   };
 
   Fetch F;
-  // ---- staging of the chunk whose inputs are in F (n tokens, flag word pa): v
-  // rows, raw k and q rows, norms, beta; cumulative decays per channel
+  // ---- staging of the chunk whose inputs are in F (n tokens, beta row and
+  // flag word pa): v rows, raw k and q rows, norms, beta; cumulative decays
+  // per channel
   auto stage_chunk = [&](int pa) {
     const int n = F.n;
     const int tid = SUMMARY ? fast::opaque(threadIdx.x) : (int)threadIdx.x, l = tid & 63;
@@ -5046,7 +5047,7 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
     if (w == 0 && l < C) {
       float bt = F.beta;
       if (D.beta_logits) bt = __builtin_amdgcn_rcpf(1.0f + __expf(-bt));
-      sm[SM_BETA * C + l] = l < n ? bt : 0.0f;
+      sm[(SM_BETA + pa) * C + l] = l < n ? bt : 0.0f;
     }
     // log2 decays of tokens 8 gq .. 8 gq + 7 of channel gc (0 past the
     // chunk's tokens), then the inclusive scan over the 32 tokens: within
@@ -5077,7 +5078,7 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
 
   fetch(F, 0);
   int ci = 0;
-  int par = 0;  // chunk parity: which flag word this chunk uses
+  int par = 0;  // chunk parity: which beta row and flag word this chunk uses
   int n = stage_chunk(par);
   fetch(F, n);  // the next chunk's inputs are in flight while this one is computed
   pf::lds_barrier();
@@ -5087,6 +5088,7 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
     // that LDS addresses are not held in registers across the loop
     const int tid = SUMMARY ? fast::opaque(threadIdx.x) : (int)threadIdx.x, l = tid & 63, q4 = l >> 4, c16 = l & 15;
     const int tt = tid >> 4, c8 = (tid & 15) * 8;
+    const float *beta = sm + (SM_BETA + par) * C;
     const bool pairwise = sm[SM_FLAG * C + par] != 0.0f;  // workgroup-uniform
     // ---- operands of token tt, channels c8 .. c8 + 7: nk k e^G and nq q e^G
     // (hi/lo, pcol order), nk k e^{G_C - G} (hi/lo), e^{G_C}; for the MFMA path
@@ -5195,7 +5197,7 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
           pp += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(pp), 0x4E, 0xF, 0xF, false));
           if (part == 0) {
             const float nks = sm[SM_NK * C + s];
-            const float av = ((sm[SM_BETA * C + t] * sm[SM_NK * C + t]) * nks) * a;
+            const float av = ((beta[t] * sm[SM_NK * C + t]) * nks) * a;
             A[t * AP + s] = av;
             if (t >= 16 && s < 16) {  // -A10 for the second block's right-hand side
               const __bf16 hi = (__bf16)(-av);
@@ -5254,7 +5256,7 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
 #pragma unroll
         for (int r = 0; r < 4; r++) {
           const int t = 16 * ti + 4 * q4 + r;
-          const float av = s0 < t ? (sm[SM_BETA * C + t] * sm[SM_NK * C + t]) * acc[r] : 0.0f;
+          const float av = s0 < t ? (beta[t] * sm[SM_NK * C + t]) * acc[r] : 0.0f;
           A[t * AP + s0] = av;
           if (blk == 1) {
             const __bf16 hi = (__bf16)(-av);
@@ -5301,8 +5303,9 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
       }
 #pragma unroll
       for (int tb = 0; tb < 2; tb++) {
-        const pf::tr4_t vr = pf::col4(VR, 16 * tb + 4 * q4, jw, c16);
-        const float4 be = *(const float4 *)(sm + SM_BETA * C + 16 * tb + 4 * q4);
+        pf::tr4_t vr = {0, 0, 0, 0};
+        if (with_v) vr = pf::col4(VR, 16 * tb + 4 * q4, jw, c16);  // VR takes the next chunk's rows beside the M pass
+        const float4 be = *(const float4 *)(beta + 16 * tb + 4 * q4);
         const float be4[4] = {be.x, be.y, be.z, be.w};
 #pragma unroll
         for (int r = 0; r < 4; r++) R[tb][r] = be4[r] * ((with_v ? pf::bf2f((uint16_t)vr[r]) : 0.0f) - ak[tb][r]);
@@ -5350,7 +5353,7 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
       for (int tb = 0; tb < 2; tb++) {
         // R_t = beta_t (v_t - (nk k e^G)_t S0), tokens 16 tb + 4 q4 .. + 3, column jw + c16
         const pf::tr4_t vr = pf::col4(VR, 16 * tb + 4 * q4, jw, c16);
-        const float4 be = *(const float4 *)(sm + SM_BETA * C + 16 * tb + 4 * q4);
+        const float4 be = *(const float4 *)(beta + 16 * tb + 4 * q4);
         const float be4[4] = {be.x, be.y, be.z, be.w};
 #pragma unroll
         for (int r = 0; r < 4; r++) R[tb][r] = be4[r] * (pf::bf2f((uint16_t)vr[r]) - ak[tb][r]);
@@ -5417,8 +5420,10 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
     state_update(S);
     if constexpr (SUMMARY) {
       if (trans) {
-        // M's columns after E's, not beside them (registers); before the
-        // next chunk's staging, which rewrites beta
+        // M's columns after E's, not beside them (registers).  No barrier
+        // lies between this pass and the staging below, and waves reach them
+        // at different times: the pass reads KG, this parity's beta, A, M, KE
+        // and EC, none of which the staging writes.
         __builtin_amdgcn_sched_barrier(0);
         ks_only(MS, false);
         solve();
@@ -5427,8 +5432,9 @@ __global__ __launch_bounds__(NT) void kda_chunk_kernel(pf::PrefillDev D) {
     }
     // The next chunk's staging, issued behind the state update's products
     // (its exponentials and scan run while they do): its rows, norms, beta
-    // and decays go to tiles that this chunk no longer reads (the update
-    // reads KE and EC only), and the barrier below orders them before use.
+    // and decays go to tiles that no wave reads past the barrier before the
+    // solve (KB, QB, VR, nk, nq, G; beta and the flag by parity), and the
+    // barrier below orders them before use.
     const int n_next = stage_chunk(par ^ 1);
     fetch(F, c_next + n_next);
     pf::lds_barrier();  // the next chunk's staging is complete, this chunk's tiles are read

@@ -93,3 +93,58 @@ def test_planned_segments_against_the_recurrence(arch, storage, monkeypatch):
     initial states) and packed ones."""
     print(f"case {arch} {storage} planned", flush=True)
     _case(arch, [1500, 70], [[700, 1500], [64, 70]], 0, monkeypatch, storage, cu_on_device=True)
+
+
+def _split(arch, lens, tokens, rate, beta, monkeypatch, repeats=1, split=True):
+    """Final states and outputs of ``repeats`` calls in segments of ``tokens``
+    (whole sequences without ``split``) with log decays of -rate (times 0 to
+    2) and the write strengths ``beta`` [T], and the float64 recurrence's."""
+    from stepquant_amd import _native as N
+    from stepquant_amd.kernels.pool import PackedStatePool
+    H, HK, K, V = 4, 4 if arch == "kda" else 2, 128, 128
+    B, T = len(lens), sum(lens)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    bits = np.full((H, K), 8)
+    pool = PackedStatePool(device_plan(make_plan(arch, bits, seed=5)), 2 * B + 1, V)
+    g = torch.Generator().manual_seed(17)
+    q, k = (torch.randn(T, HK, K, generator=g).to(torch.bfloat16) for _ in range(2))
+    v = torch.randn(T, H, V, generator=g).to(torch.bfloat16)
+    gate = -rate * 2 * torch.rand((T, H, K) if arch == "kda" else (T, H), generator=g)
+    beta = torch.as_tensor(beta, dtype=torch.float32).reshape(T, 1) * (.9 + .1 * torch.rand(T, H, generator=g))
+    init = torch.arange(1, B + 1)
+    pool.encode((torch.randn(B, H, K, V, generator=g) * .5).to(dev()), init.to(dev()))
+    torch.cuda.synchronize()
+    plan, lay = make_plan(arch, bits, seed=5), O.layout(make_plan(arch, bits, seed=5), V)
+    S0 = O.decode_page(pool.data.cpu().numpy(), init.numpy(), plan, lay, V).astype(np.float64)
+    segments = N.PrefillSegments(tokens, -(-max(lens) // tokens),
+                                 2 * (T // tokens + B) * H * K * V * 4, None) if split else N.PrefillSegments()
+    monkeypatch.setattr(N, "prefill_plan", lambda desc, offsets, cus=0: segments)
+    pool.keep_prefill_states = True
+    ck = np.asarray(lens).reshape(B, 1)
+    inputs = [t.to(dev()) for t in (q, k, v, gate, beta)]
+    got = []
+    for _ in range(repeats):
+        out = pool.extend(*inputs, init, torch.from_numpy(cu), checkpoints=torch.tensor(ck),
+                          checkpoint_slots=torch.arange(B + 1, 2 * B + 1).reshape(B, 1), init_slots=init,
+                          normalize=True, scale=K ** -.5)
+        torch.cuda.synchronize()
+        got.append((out.cpu(), pool.last_prefill[-1].cpu().reshape(B, H, K, V)))
+    ref_out, _, ref_states = O.prefill(q.float().numpy(), k.float().numpy(), v.float().numpy(), gate.numpy(),
+                                       beta.numpy(), S0, cu, ck, normalize=True, scale=K ** -.5)
+    return got, ref_out, ref_states
+
+
+@pytest.mark.parametrize("arch,tokens", [("gdn", 64), ("gdn", 192), ("kda", 32), ("kda", 96), ("kda", 224)])
+def test_segments_with_write_strengths_that_change_by_chunk(arch, tokens, monkeypatch):
+    """Write strengths of .98 and .02 in turn from chunk to chunk: a wave that
+    scales a chunk's rows with the next chunk's strengths is far off.  Equal
+    calls give equal bits."""
+    print(f"case {arch} tokens={tokens}", flush=True)
+    lens = [960, 417]
+    chunk = 64 if arch == "gdn" else 32
+    beta = np.concatenate([np.where(np.arange(t) // chunk % 2, .98, .02) for t in lens])
+    got, ref_out, ref_states = _split(arch, lens, tokens, 1e-3, beta, monkeypatch, repeats=6)
+    for out, states in got:
+        assert torch.equal(out, got[0][0]) and torch.equal(states, got[0][1])
+    check_prefill(got[0][0], ref_out, f"{arch} tokens={tokens}")
+    check_states(got[0][1].numpy(), ref_states)
