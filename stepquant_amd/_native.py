@@ -176,9 +176,10 @@ def step_entry(name: str):
     fn = _step_entries.get(name)
     if fn is not None:
         return fn
-    fn = _step_entries[name] = lib()[name]  # a function object of its own: lib()'s keeps its prototype
+    fn = lib()[name]  # a function object of its own: lib()'s keeps its prototype
     fn.restype = ctypes.c_int
     fn.argtypes = [_P, ctypes.c_char_p] + ([PP(Scratch), _P] if name == "sq_decode_readout" else [_P])
+    _step_entries[name] = fn  # with its prototype: another thread may call it from here on
     return fn
 
 

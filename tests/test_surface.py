@@ -203,3 +203,20 @@ def test_constructor_signature_matches_the_reference_order():
     sig = re.search(r"PackedStatePool\(plan, slots, value_dim=128,\s+writeback_stream=None,\s+"
                     r"writeback_workspace=None,\s+writeback_chunk=64,\s+storage=\"packed\"\)", doc)
     assert sig, "INTEGRATION.md documents the constructor in this order"
+
+
+@pytest.mark.parametrize("name", ["sq_decode_step", "sq_decode_readout", "sq_format_step"])
+def test_step_entries_are_published_with_their_prototype(name, monkeypatch):
+    """A thread that finds an entry may call it at once: without its argument
+    types ctypes would pass the pool's address as a 32-bit int."""
+    from stepquant_amd import _native as N
+
+    class Entry:
+        def __setattr__(self, key, value):
+            assert name not in N._step_entries, f"published before {key} is set"
+            object.__setattr__(self, key, value)
+
+    monkeypatch.setattr(N, "_step_entries", {})
+    monkeypatch.setattr(N, "lib", lambda: {name: Entry()})
+    fn = N.step_entry(name)
+    assert N._step_entries[name] is fn and len(fn.argtypes) == (4 if name == "sq_decode_readout" else 3)
