@@ -292,9 +292,12 @@ int sq_copy_slots(const sq_pool *pool, const void *src, const void *dst, int32_t
 /*
  * The same copy of at most SQ_COPY_DIRECT_PAGES pages without `temp`: one
  * kernel holds each byte range of all the pages between reading and writing
- * it.  Page sizes must be even and the pool 16-byte aligned (SQ_EINVAL
- * otherwise, and above that count).  Safe under capture and on any number
- * of streams.
+ * it.  Page sizes must be even and at most 2^31 bytes and the pool 16-byte
+ * aligned (SQ_EINVAL otherwise, and above that count).  Page sizes that are
+ * no multiple of 16 are read in aligned windows, up to 14 bytes into the
+ * slack behind the last page (sq_pool.data); sq_copy_slots and
+ * sq_copy_slots_static take the same kernel for such lists.  Safe under
+ * capture and on any number of streams.
  */
 #define SQ_COPY_DIRECT_PAGES 256
 int sq_copy_slots_direct(const sq_pool *pool, const void *src, const void *dst, int32_t slots_dtype, int64_t n,

@@ -202,6 +202,12 @@ def pool_flags(bits, head_meta, columns, H, K, V, group, kda, storage, page_byte
     return rc
 
 
+def copies_directly(pool: Pool) -> bool:
+    """Whether sq_copy_slots_direct takes the pool's pages; others go through a
+    staging buffer."""
+    return pool.data % 16 == 0 and pool.page_bytes % 2 == 0 and pool.page_bytes <= 1 << 31
+
+
 def prefill_plan(pool: Pool, cu_seqlens: torch.Tensor, cus: int = 0) -> PrefillSegments:
     """sq_prefill_plan of host int32 sequence offsets."""
     segments = PrefillSegments()

@@ -6628,8 +6628,10 @@ int static_scratch(uint8_t **out) {
   return 0;
 }
 
+// (a launch has fewer than 2^32 threads: pages up to 2^31 bytes, 240 or more a workgroup, stay far below)
 bool copy_is_direct(const sq_pool *pool, int64_t n) {
-  return n <= COPY_PAGES && pool->page_bytes > 0 && pool->page_bytes % 2 == 0 && ((uintptr_t)pool->data & 15) == 0;
+  return n <= COPY_PAGES && pool->page_bytes > 0 && pool->page_bytes <= (int64_t)1 << 31 && pool->page_bytes % 2 == 0 &&
+         ((uintptr_t)pool->data & 15) == 0;
 }
 
 // temp may be NULL for lists that copy_kernel takes
@@ -6644,12 +6646,10 @@ int launch_copy(const sq_pool *pool, const void *src, const void *dst, int32_t s
       hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), aligned ? 0 : 16 * 256 * windows, stream,
                          pool->data, pool->page_bytes, pool->num_slots, src, dst, slots_dtype, (int)n, lr_log);
     };
-    if (blocks < (int64_t)1 << 31) {
-      if (per > 4) launch(aligned ? copy_kernel<true, 16> : copy_kernel<false, 16>, COPY_WINDOWS / 256);
-      else if (per > 1) launch(aligned ? copy_kernel<true, 4> : copy_kernel<false, 4>, 4);
-      else launch(aligned ? copy_kernel<true, 1> : copy_kernel<false, 1>, 1);
-      return check_launch("copy_kernel");
-    }
+    if (per > 4) launch(aligned ? copy_kernel<true, 16> : copy_kernel<false, 16>, COPY_WINDOWS / 256);
+    else if (per > 1) launch(aligned ? copy_kernel<true, 4> : copy_kernel<false, 4>, 4);
+    else launch(aligned ? copy_kernel<true, 1> : copy_kernel<false, 1>, 1);
+    return check_launch("copy_kernel");
   }
   unsigned gx = (unsigned)((pool->page_bytes + 255) / 256);
   if (gx > 1024) gx = 1024;

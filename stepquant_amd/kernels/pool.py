@@ -624,7 +624,7 @@ class PackedStatePool:
         dst = _indices(destination, self.device).to(torch.int64)
         if src.numel() != dst.numel():
             raise ValueError("copy needs as many destination slots as source slots")
-        if 0 < src.numel() <= N.COPY_DIRECT_PAGES and self.page_bytes % 2 == 0:
+        if 0 < src.numel() <= N.COPY_DIRECT_PAGES and N.copies_directly(self._desc):
             N.check(N.lib().sq_copy_slots_direct(self._desc, N.ptr(src), N.ptr(dst), N.I64, src.numel(),
                                                  N.stream_handle()), "copy")
         elif src.numel():

@@ -220,3 +220,27 @@ def test_step_entries_are_published_with_their_prototype(name, monkeypatch):
     monkeypatch.setattr(N, "lib", lambda: {name: Entry()})
     fn = N.step_entry(name)
     assert N._step_entries[name] is fn and len(fn.argtypes) == (4 if name == "sq_decode_readout" else 3)
+
+
+@pytest.mark.parametrize("data,page_bytes,n,entry", [
+    (4096, 1040, 3, "sq_copy_slots_direct"), (4096, 1042, 256, "sq_copy_slots_direct"),
+    (4104, 1040, 3, "sq_copy_slots"), (4098, 1042, 3, "sq_copy_slots"),  # pages not on a 16-byte boundary
+    (4096, 1041, 3, "sq_copy_slots"), (4096, 1040, 257, "sq_copy_slots")])
+def test_copy_takes_every_pool(data, page_bytes, n, entry, monkeypatch):
+    """Pools that the one-kernel copy refuses are copied through a staging buffer."""
+    from stepquant_amd import _native as N
+    from stepquant_amd.kernels.pool import PackedStatePool
+    called = []
+
+    class Lib:
+        def __getattr__(self, name):
+            return lambda *args: called.append(name) or 0
+
+    pool = object.__new__(PackedStatePool)
+    pool.device, pool.page_bytes = torch.device("cpu"), page_bytes
+    pool._desc = N.Pool(data=data, page_bytes=page_bytes, num_slots=600)
+    pool.wait = lambda: None
+    monkeypatch.setattr(N, "lib", Lib)
+    monkeypatch.setattr(N, "stream_handle", lambda *a: None)
+    pool.copy(torch.arange(n), torch.arange(300, 300 + n))
+    assert called == [entry]
