@@ -259,6 +259,9 @@ int sq_prefill(const sq_pool *pool, const sq_prefill_args *args, void *stream);
  * sequence, and the device workspace they need.  The caller allocates it
  * (16-byte aligned), sets `workspace` and hands the plan, with the same
  * cu_seqlens, to sq_prefill_split; NULL or tokens == 0 there is sq_prefill.
+ * A plan made for other offsets is slower, not wrong: the last segment of a
+ * sequence runs to its end, and sequences without room in the workspace stay
+ * whole.
  * Three launches: every segment's effect on a state (S_end = M S_start + E,
  * both fp32), the start states from them, the segments themselves.
  * No counterpart in the reference.

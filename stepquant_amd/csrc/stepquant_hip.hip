@@ -3764,30 +3764,42 @@ struct PrefillDev {
   float scale;
   int page_init;  // 1: initial states decoded from the pages of pi.slots inside the kernel
   PageInit pi;
-  // sequences cut into segments of seg tokens (0: whole sequences); seg_state
-  // and seg_trans hold [segment slot][H][K][V] f32 (see Segment)
-  int seg;
+  // sequences cut into segments of seg tokens (0: whole sequences), at most
+  // seg_count each; seg_state and seg_trans hold [seg_slots][H][K][V] f32 (see
+  // Segment)
+  int seg, seg_count, seg_slots;
   float *seg_state, *seg_trans;
 };
 
 // One segment of a sequence: tokens t0 .. t0 + len - 1 of the packed rows,
 // start tokens into its sequence.  Its workspace slot t0_seq / seg + b + s is
 // distinct for every (b, s): a sequence takes at most ceil(len / seg) slots
-// and the next one starts at least floor(len / seg) + 1 further.
+// and the next one starts at least floor(len / seg) + 1 further.  The last of
+// a sequence's segments runs to its end, whatever the plan's count, and a
+// sequence whose slots would lie past the workspace stays whole: segments
+// planned for other lengths cost time, never tokens or memory.
 struct Segment {
   int t0, len, start, slot;
   bool last;  // of its sequence
 };
+// segments of the sequence of len tokens whose first slot is `slot`
+__device__ __forceinline__ int segments_of(const PrefillDev &D, int len, int slot) {
+  if (len <= 0) return 0;
+  int n = (int)((unsigned)(len - 1) / (unsigned)D.seg) + 1;
+  n = n < D.seg_count ? n : D.seg_count;
+  return slot >= 0 && slot + n - 1 <= D.seg_slots ? n : 1;  // (the last one takes no slot)
+}
 __device__ __forceinline__ Segment segment_of(const PrefillDev &D, int b, int s) {
   Segment r;
   const int t0 = __builtin_amdgcn_readfirstlane(D.cu[b]);
   const int len = __builtin_amdgcn_readfirstlane(D.cu[b + 1]) - t0;
   if (D.seg == 0) return Segment{t0, len, 0, 0, true};
+  const int first = (int)((unsigned)t0 / (unsigned)D.seg) + b, n = segments_of(D, len, first);
   r.start = s * D.seg;
   r.t0 = t0 + r.start;
-  r.len = len - r.start < D.seg ? len - r.start : D.seg;
-  r.slot = (int)((unsigned)t0 / (unsigned)D.seg) + b + s;
-  r.last = r.start + D.seg >= len;
+  r.len = s < n - 1 ? D.seg : s == n - 1 ? len - r.start : 0;
+  r.slot = first + s;
+  r.last = s >= n - 1;
   return r;
 }
 
@@ -4630,7 +4642,7 @@ __global__ __launch_bounds__(NT) void segment_combine_kernel(PrefillDev D) {
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, q4 = l >> 4, c16 = l & 15;
   const Segment first = segment_of(D, b, 0);
   const int len = __builtin_amdgcn_readfirstlane(D.cu[b + 1]) - first.t0;
-  const int n = len > 0 ? (len - 1) / D.seg : 0;  // summaries 0 .. n - 1: segments but the last
+  const int n = segments_of(D, len, first.slot) - 1;  // summaries 0 .. n - 1: segments but the last
   if (n < 2) return;
   const int64_t step = (int64_t)H * PKD * PV;
   float *state = D.seg_state + ((int64_t)first.slot * H + h) * PKD * PV + jw + (16 * w + 4 * q4) * PV + c16;
@@ -7087,6 +7099,8 @@ int sq_prefill_split(const sq_pool *pool, const sq_prefill_args *a, const sq_pre
   D.pi.slots_dtype = a->slots_dtype;
   D.pi.ng = pool->group >= 32 ? 128 / pool->group : 1;
   D.seg = split ? sg->tokens : 0;
+  D.seg_count = split ? sg->count : 1;
+  D.seg_slots = split ? (int)(sg->workspace_bytes / (2 * (int64_t)H * 128 * 128 * sizeof(float))) : 0;
   D.seg_state = split ? (float *)sg->workspace : nullptr;
   D.seg_trans = split ? D.seg_state + sg->workspace_bytes / (2 * sizeof(float)) : nullptr;
   const unsigned tiles = (unsigned)(a->batch * H), count = split ? (unsigned)sg->count : 1u;

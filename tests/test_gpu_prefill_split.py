@@ -95,10 +95,11 @@ def test_planned_segments_against_the_recurrence(arch, storage, monkeypatch):
     _case(arch, [1500, 70], [[700, 1500], [64, 70]], 0, monkeypatch, storage, cu_on_device=True)
 
 
-def _split(arch, lens, tokens, rate, beta, monkeypatch, repeats=1, split=True):
+def _split(arch, lens, tokens, rate, beta, monkeypatch, repeats=1, planned=None):
     """Final states and outputs of ``repeats`` calls in segments of ``tokens``
-    (whole sequences without ``split``) with log decays of -rate (times 0 to
-    2) and the write strengths ``beta`` [T], and the float64 recurrence's."""
+    (0: whole sequences) planned for the lengths ``planned`` (default: the
+    call's own) with log decays of -rate (times 0 to 2) and the write strengths
+    ``beta`` [T], and the float64 recurrence's."""
     from stepquant_amd import _native as N
     from stepquant_amd.kernels.pool import PackedStatePool
     H, HK, K, V = 4, 4 if arch == "kda" else 2, 128, 128
@@ -116,8 +117,10 @@ def _split(arch, lens, tokens, rate, beta, monkeypatch, repeats=1, split=True):
     torch.cuda.synchronize()
     plan, lay = make_plan(arch, bits, seed=5), O.layout(make_plan(arch, bits, seed=5), V)
     S0 = O.decode_page(pool.data.cpu().numpy(), init.numpy(), plan, lay, V).astype(np.float64)
-    segments = N.PrefillSegments(tokens, -(-max(lens) // tokens),
-                                 2 * (T // tokens + B) * H * K * V * 4, None) if split else N.PrefillSegments()
+    planned = lens if planned is None else planned
+    segments = N.PrefillSegments(tokens, -(-max(planned) // tokens),
+                                 2 * (sum(planned) // tokens + B) * H * K * V * 4, None) if tokens else \
+        N.PrefillSegments()
     monkeypatch.setattr(N, "prefill_plan", lambda desc, offsets, cus=0: segments)
     pool.keep_prefill_states = True
     ck = np.asarray(lens).reshape(B, 1)
@@ -146,5 +149,20 @@ def test_segments_with_write_strengths_that_change_by_chunk(arch, tokens, monkey
     got, ref_out, ref_states = _split(arch, lens, tokens, 1e-3, beta, monkeypatch, repeats=6)
     for out, states in got:
         assert torch.equal(out, got[0][0]) and torch.equal(states, got[0][1])
+    check_prefill(got[0][0], ref_out, f"{arch} tokens={tokens}")
+    check_states(got[0][1].numpy(), ref_states)
+
+
+@pytest.mark.parametrize("arch,tokens,lens,planned", [
+    ("gdn", 64, [960, 417], [65, 1]),      # the first in two segments, the second without a slot of its own
+    ("gdn", 128, [100, 961], [961, 100]),  # slots for both, the long one elsewhere
+    ("gdn", 64, [1, 700], [700, 1]),
+    ("kda", 32, [960, 417], [65, 1]),
+    ("kda", 96, [417, 960, 5], [961, 1, 1])])
+def test_segments_planned_for_other_lengths(arch, tokens, lens, planned, monkeypatch):
+    """A plan that belongs to other offsets leaves no token out."""
+    print(f"case {arch} tokens={tokens} {lens} planned for {planned}", flush=True)
+    beta = np.full(sum(lens), .5)
+    got, ref_out, ref_states = _split(arch, lens, tokens, 1e-3, beta, monkeypatch, planned=planned)
     check_prefill(got[0][0], ref_out, f"{arch} tokens={tokens}")
     check_states(got[0][1].numpy(), ref_states)
