@@ -4629,15 +4629,24 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
 // state after segment s, S_{s+1} = M_s S_s + E_s for s = 1 .. the last but
 // one.  State columns are independent: a workgroup takes 16 columns of one
 // (sequence, head), wave w the rows 16 w .. 16 w + 15, with the 128 x 16 state
-// handed from wave to wave through LDS as hi/lo bf16 (products hi*hi + hi*lo
-// + lo*hi, as in the recurrence).  Bound by the loads of M, 64 KB a step:
-// those of the next two segments are in flight behind each step's products,
-// and the eight workgroups that read one M sit on one XCD (grid x is
-// sequences x heads, dealt to the XCDs in turn).
-constexpr int CB_PITCH = 136;  // elements of a column in the LDS copy of the state
+// handed from wave to wave through LDS.  All of it in fp32
+// (v_mfma_f32_16x16x4_f32): M carries the state's decay, which a whole
+// sequence multiplies in fp32 too, so operands in fewer bits would add their
+// rounding to the whole state once a segment.  (Slowly forgetting states, T =
+// 2048 in 32 segments, relative error to float64: 7.0e-7 uncut, 9.6e-7 here,
+// 2.1e-5 with hi/lo bf16 pairs.)
+// Bound by the loads of M, 64 KB a step: those of the next two segments are
+// in flight behind each step's products, and the eight workgroups that read
+// one M sit on one XCD (grid x is sequences x heads, dealt to the XCDs in
+// turn).
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
+  // lane l holds A[l % 16][l / 16] and B[l / 16][l % 16]; the result as mfma's
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+constexpr int CB_PITCH = 132;  // floats of a column in the LDS copy of the state
 __global__ __launch_bounds__(NT) void segment_combine_kernel(PrefillDev D) {
 #pragma clang fp contract(off)
-  __shared__ __align__(16) uint16_t st[2][2][16 * CB_PITCH];  // [buffer][hi, lo][column][row]
+  __shared__ __align__(16) float st[2][16 * CB_PITCH];  // [buffer][column][row]
   const int H = D.H, h = blockIdx.x % H, b = blockIdx.x / H, jw = 16 * blockIdx.y;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, q4 = l >> 4, c16 = l & 15;
   const Segment first = segment_of(D, b, 0);
@@ -4647,14 +4656,12 @@ __global__ __launch_bounds__(NT) void segment_combine_kernel(PrefillDev D) {
   const int64_t step = (int64_t)H * PKD * PV;
   float *state = D.seg_state + ((int64_t)first.slot * H + h) * PKD * PV + jw + (16 * w + 4 * q4) * PV + c16;
   const float *trans = D.seg_trans + ((int64_t)first.slot * H + h) * PKD * PV + (16 * w + c16) * PV + 4 * q4;
-  f32x4 m[2][4][2];  // of two segments: row 16 w + c16, columns 32 kb + 16 i + 4 q4 .. + 3
-  f32x4 e[2], x;     // rows 16 w + 4 q4 + r of column jw + c16
-  auto load = [&](int s, f32x4 (&mm)[4][2], f32x4 &ee) {
+  f32x4 m[2][8];  // of two segments: row 16 w + c16, columns 16 i + 4 q4 .. + 3
+  f32x4 e[2], x;  // rows 16 w + 4 q4 + r of column jw + c16
+  auto load = [&](int s, f32x4 (&mm)[8], f32x4 &ee) {
     const int64_t at = step * (s < n ? s : n - 1);
 #pragma unroll
-    for (int kb = 0; kb < 4; kb++)
-#pragma unroll
-      for (int i = 0; i < 2; i++) mm[kb][i] = *(const f32x4 *)(trans + at + 32 * kb + 16 * i);
+    for (int i = 0; i < 8; i++) mm[i] = *(const f32x4 *)(trans + at + 16 * i);
 #pragma unroll
     for (int r = 0; r < 4; r++) ee[r] = state[at + r * PV];
   };
@@ -4662,29 +4669,26 @@ __global__ __launch_bounds__(NT) void segment_combine_kernel(PrefillDev D) {
   for (int r = 0; r < 4; r++) x[r] = state[r * PV];
   load(1, m[0], e[0]);
   load(2, m[1], e[1]);
-  auto one = [&](int s, f32x4 (&mm)[4][2], f32x4 &ee, int buf) {
-    uint2 hi, lo;
-    split2(x[0], x[1], hi.x, lo.x);
-    split2(x[2], x[3], hi.y, lo.y);
-    const int put = c16 * CB_PITCH + pcol(16 * w + 4 * q4);  // rows in split8's slot order
-    *(uint2 *)(st[buf][0] + put) = hi;
-    *(uint2 *)(st[buf][1] + put) = lo;
-    bf16x8 mh[4], ml[4];
+  auto one = [&](int s, f32x4 (&mm)[8], f32x4 &ee, int buf) {
+    *(f32x4 *)(st[buf] + c16 * CB_PITCH + 16 * w + 4 * q4) = x;
+    f32x4 a[8];
 #pragma unroll
-    for (int kb = 0; kb < 4; kb++) split8(mm[kb][0], mm[kb][1], mh[kb], ml[kb]);
+    for (int i = 0; i < 8; i++) a[i] = mm[i];
     x = ee;
     load(s + 2, mm, ee);
     // one barrier a segment: the other buffer's readers are past theirs
     lds_barrier();
-    f32x4 y = {0.f, 0.f, 0.f, 0.f};  // two chains: blocks 0, 1 and 2, 3
+    f32x4 y = {0.f, 0.f, 0.f, 0.f};  // two chains: columns 0-63 and 64-127
 #pragma unroll
-    for (int kb = 0; kb < 4; kb++) {
-      const int at = (c16 * CB_PITCH + 32 * kb + 8 * q4) * 2;
-      const bf16x8 sh = ld8((const uint8_t *)st[buf][0], at), sl = ld8((const uint8_t *)st[buf][1], at);
-      f32x4 &acc = kb < 2 ? x : y;
-      acc = mfma(mh[kb], sh, acc);
-      acc = mfma(mh[kb], sl, acc);
-      acc = mfma(ml[kb], sh, acc);
+    for (int i = 0; i < 4; i++) {
+      // product r of a block takes the columns 16 i + 4 q4 + r, one per lane row
+      const f32x4 s0 = *(const f32x4 *)(st[buf] + c16 * CB_PITCH + 16 * i + 4 * q4);
+      const f32x4 s1 = *(const f32x4 *)(st[buf] + c16 * CB_PITCH + 64 + 16 * i + 4 * q4);
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        x = mfma_f32(a[i][r], s0[r], x);
+        y = mfma_f32(a[i + 4][r], s1[r], y);
+      }
     }
 #pragma unroll
     for (int r = 0; r < 4; r++) {

@@ -3,8 +3,8 @@
 Gates that forget slowly (down to 1e-3 a token) carry the state across
 segments, so an error in a segment's transition or start state shows.  Bars
 as for whole sequences: states rtol 1e-3 / atol 1e-4 of the float64
-recurrence, outputs rtol 2^-8 / atol 1e-4; the transitions add products of
-the same hi/lo operands (~2^-17 relative), one per segment.
+recurrence, outputs rtol 2^-8 / atol 1e-4; the segments' states are chained
+in fp32, which adds about 2^-24 relative a segment.
 """
 import numpy as np
 import pytest
@@ -166,3 +166,22 @@ def test_segments_planned_for_other_lengths(arch, tokens, lens, planned, monkeyp
     got, ref_out, ref_states = _split(arch, lens, tokens, 1e-3, beta, monkeypatch, planned=planned)
     check_prefill(got[0][0], ref_out, f"{arch} tokens={tokens}")
     check_states(got[0][1].numpy(), ref_states)
+
+
+@pytest.mark.parametrize("arch", ["gdn", "kda"])
+@pytest.mark.parametrize("rate,strength", [(1e-5, .01), (1e-4, .1), (1e-3, .5)])
+def test_segments_carry_the_state_as_whole_sequences_do(arch, rate, strength, monkeypatch):
+    """States that forget little, through 32 segments: as near to float64 as
+    the uncut sequence's, plus one fp32 rounding (2^-24) of the state a
+    segment.  (Operands of 16 bits in the chain would add 2^-18 a segment.)"""
+    lens, beta = [2048], np.full(2048, strength)
+
+    def error(tokens):
+        got, _, ref = _split(arch, lens, tokens, rate, beta, monkeypatch)
+        return np.linalg.norm(got[0][1].double().numpy() - ref) / np.linalg.norm(ref)
+
+    whole = error(0)
+    for tokens in (64, 320):
+        split, bound = error(tokens), 1.25 * whole + -(-2048 // tokens) * 2 ** -24
+        print(f"case {arch} rate={rate} tokens={tokens}: {split:.2e}, whole {whole:.2e}", flush=True)
+        assert split <= bound
