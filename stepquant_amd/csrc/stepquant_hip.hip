@@ -3892,6 +3892,18 @@ typedef short bf16x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
+// An accumulator that a product of the other shape continues (16 x 16 x 32 to
+// 16 x 16 x 16): 8 wait states after the last product, what a vector
+// instruction that reads its result needs.  The compiler leaves none, as
+// between products of one shape, whose accumulator is forwarded.  Built
+// without this, the two were one issue slot apart at a single place of all
+// kernels (D_3 of the segment summaries), and those rows alone differed from
+// run to run; pairs at least 4 slots apart have always repeated exactly.  One
+// wait a chunk: no measurable time.
+__device__ __forceinline__ f32x4 other_shape(f32x4 x) {
+  asm("s_nop 7" : "+v"(x));
+  return x;
+}
 __device__ __forceinline__ bf16x8 ld8(const uint8_t *lds, int byte) { return *(const bf16x8 *)(lds + byte); }
 __device__ __forceinline__ bf16x4 ld4(const uint8_t *lds, int byte) { return *(const bf16x4 *)(lds + byte); }
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -4467,7 +4479,6 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
     auto delta_solve = [&](const f32x4 (&R)[4]) {
       const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
       bf16x4 xh[4], xl[4];
-      f32x4 c0, c1;
       // acc + M[16 i .. 16 i + 15][16 k .. 16 k + 15] x (hi/lo pairs hi*hi + hi*lo + lo*hi)
       auto mone = [&](int i, int k, bf16x4 bh, bf16x4 bl, f32x4 acc) {
         const int o = ((16 * i + c16) * P72 + pcol(16 * k + 4 * q4)) * 2;
@@ -4480,24 +4491,19 @@ __global__ __launch_bounds__(NT) void prefill_kernel(PrefillDev D) {
       auto mpair = [&](int i, f32x4 acc) {
         const int o = ((16 * i + c16) * P72 + 8 * q4) * 2;
         const bf16x8 mh = ld8(Tb, o), ml = ld8(Tb, PC * P72 * 2 + o);
-        c0 = mfma(mh, ph01, acc);
-        c1 = mfma(mh, pl01, c0);
-        return mfma(ml, ph01, c1);
+        acc = mfma(mh, ph01, acc);
+        acc = mfma(mh, pl01, acc);
+        return mfma(ml, ph01, acc);
       };
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         f32x4 acc = R[i];
         if (i == 1) acc = mone(1, 0, xh[0], xl[0], acc);
         if (i >= 2) acc = mpair(i, acc);
-        if (i == 3) acc = mone(3, 2, xh[2], xl[2], acc);
+        if (i == 3) acc = mone(3, 2, xh[2], xl[2], other_shape(acc));
         bf16x4 ah, al;
         split4x(acc, ah, al);
-        f32x4 d = mone(i, i, ah, al, zero);
-        // the chain's accumulator inputs stay allocated until its result: a
-        // register of theirs rewritten a few instructions after the product
-        // that reads it (nothing else held it) gave wrong rows of D_3 in the
-        // summary kernel, differently from run to run
-        if (i >= 2) asm volatile("" : "+v"(d) : "v"(c0), "v"(c1), "v"(R[i]));
+        const f32x4 d = mone(i, i, ah, al, zero);
         split4x(d, xh[i], xl[i]);
         if (i == 1) {
           ph01 = cat8(xh[0], xh[1]);
