@@ -1826,6 +1826,15 @@ __device__ __forceinline__ void store_out(const PoolDev &P, const StepDev &S, co
 typedef const __attribute__((address_space(1))) void *gptr_t;
 typedef __attribute__((address_space(3))) void *lptr_t;
 
+// Workgroup barrier behind direct global-to-LDS loads.  A barrier alone orders
+// LDS accesses; that a wave's direct loads have landed follows only from its
+// own wait, placed here instead of left to a later load that it happens to use
+// first.
+__device__ __forceinline__ void staged_barrier() {
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), the other counters free
+  __syncthreads();
+}
+
 template <int CH>
 __device__ __forceinline__ void stage_async(const Ctx &C, int row_chunks, bool cols) {
   const int wv = C.tid >> 6;
@@ -3452,7 +3461,7 @@ __device__ __forceinline__ void body(const PoolDev &P, const StepDev &S, Lds &T,
     const uint64_t m = __ballot(width == 16);
     if (l == 0) T.piv[wave - 2] = m;
   }
-  __syncthreads();
+  fast::staged_barrier();
   const bool pivots = KIND == KDA_ROWS ? (T.piv[0] | T.piv[1]) != 0 : KIND == GDN_PIV;
 
   // ---- this lane's values, x = ((r d) c_j) z (pivots: half * d)
@@ -6131,7 +6140,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DSQ ? 3 : 4
   } else {
     sz[i] = make_float2(os, oz);
   }
-  __syncthreads();
+  if constexpr (CODES) fast::staged_barrier();
+  else __syncthreads();
 
   // ---- x = ((code - z) s) d, k^T x
   float kr[4] = {0.f, 0.f, 0.f, 0.f};
