@@ -3568,6 +3568,9 @@ __device__ __forceinline__ void body(const PoolDev &P, const StepDev &S, Lds &T,
         hv.x = f2h(x[r][0]) | (f2h(x[r][1]) << 16);
         hv.y = f2h(x[r][2]) | (f2h(x[r][3]) << 16);
         *(uint2 *)(page + T.pivpos[rg + 8 * r] + 2 * j0) = hv;
+        // no part in the column statistics, which an infinite value times its zero factor would enter as NaN
+#pragma unroll
+        for (int c = 0; c < 4; c++) x[r][c] = 0.0f;
       }
     }
   }

@@ -74,3 +74,49 @@ def test_byte_kernel_matches_the_general_one(arch, group, dtype, gate, scale):
     assert torch.equal(outs[0], outs[1]), "outputs differ from the general kernel's"
     assert not outs[0][1].any()
     assert torch.equal(pools[0].data, pools[1].data), "pages differ from the general kernel's"
+
+
+def test_infinite_pivots_stay_out_of_the_column_scales():
+    """A pivot value past the fp16 range comes back as infinity.  The pages stay
+    the general kernel's: its column's integer rows saturate, and no scale
+    turns NaN."""
+    from stepquant_amd.kernels.pool import PackedStatePool
+    rng = np.random.default_rng(6)
+    H, K, V, B = 2, 128, 128, 2
+    bits = rng.choice([4, 6, 8], (H, K))
+    bits[0, [3, 70]] = 16
+    oplan = make_plan("kda", bits, seed=4)
+    pools = [PackedStatePool(device_plan(oplan), B + 1, V, writeback_stream=torch.cuda.Stream(), storage="byte")
+             for _ in range(2)]
+    assert pools[0]._desc.flags == N.POOL_FAST_BYTE128
+    pools[1]._desc.flags = 0  # the general kernel
+    g = torch.Generator().manual_seed(8)
+    slots = torch.tensor([2, 1], device=dev())
+    x = torch.randn(B, H, K, V, generator=g) * .05
+    for p in pools:
+        p.encode(x.to(dev()), slots)
+        p.wait()
+    torch.cuda.synchronize()
+    at = [int(pools[0].offsets[row]) + 2 * j for row, j in ((3, 0), (3, 65), (70, 66), (70, 127))]
+    for p in pools:
+        for e in at:
+            p.data[:, e + 1] = 0x7c  # the halves' high bytes: infinity
+            p.data[:, e] = 0
+    q, k, v = (torch.randn(B, H * K, generator=g).to(dev()) for _ in range(3))
+    gate = -torch.rand(B, H, K, generator=g).to(dev())
+    beta = torch.rand(B, H, generator=g).to(dev())
+    torch.cuda.synchronize()
+    pages = []
+    for p in pools:
+        p.step(q, k, v, gate, beta, slots, normalize=True, scale=K ** -.5)
+        p.wait()
+        torch.cuda.synchronize()
+        for e in at:  # infinity less infinity: NaN, of either payload
+            half = p.data[slots, e:e + 2].contiguous().view(torch.float16)
+            assert torch.isnan(half).all()
+            p.data[:, e:e + 2] = 0
+        pages.append(p.data[slots])
+    column = int(pools[0].columns[0])
+    scales = [d[:, column:column + 2 * V].contiguous().view(torch.float16) for d in pages]
+    assert torch.isfinite(scales[1]).all() and torch.equal(scales[0], scales[1])
+    assert torch.equal(pages[0], pages[1])
