@@ -6985,20 +6985,25 @@ int sq_prefill_plan(const sq_pool *pool, const int32_t *cu, int64_t batch, int32
   const int64_t H = pool->heads;
   if (batch == 0 || H < 1 || batch * H > cus) return 0;
   // Time of a call whose workgroups all fit the device at once (one per
-  // compute unit), measured in microseconds: whole sequences take 6.1 a
+  // compute unit), measured in microseconds.  GDN: whole sequences take 6.1 a
   // 64-token chunk (32 workgroups), one after the other; cut into P segments,
   // every segment's summary and full pass take 7.9 + 7.7 a chunk (256
   // workgroups) over longest / P tokens, and the combine 2.5 a segment.
   // (B = 1, T = 8192, 32 heads: 785 us whole, 127 + 125 + 20 us in 8
-  // segments.)  KDA, per 32-token chunk: 8.2 whole, 9.5 + 9.1 split (three
-  // sequences of 3001, 1456 and 2411 tokens, 32 heads: 771 us whole, 304 +
-  // 292 + 15 us in 3 segments).  A split that saves less than 15% is not
-  // taken.
-  const double whole_chunk = pool->kda ? 8.2 : 6.1, split_chunk = pool->kda ? 18.6 : 15.6, step = 2.5, extra = 8.0;
+  // segments.)  A split that saves less than 15% is not taken: cut calls of
+  // 1024 tokens and more (1 to 7 sequences, 4 to 64 heads) run 1.1 to 3.1 times
+  // as fast, the shortest that are cut, 640 tokens, 0.92 to 1.17 (mean 1.04).
+  // KDA, per 32-token chunk, fitted to 60 calls of 256 to 1500 tokens (rms 5):
+  // 8.0 whole; 17.4 cut, 2.0 a segment, .071 a workgroup (the traffic of the
+  // segments' states).  The line lies 3% below whole: 256 tokens in segments
+  // of 32 run 1.05 to 1.19 times as fast and are cut, in segments of 64 (160 to
+  // 256 workgroups) 0.93 to 1.02 and are not.
+  const double whole_chunk = pool->kda ? 8.0 : 6.1, split_chunk = pool->kda ? 17.4 : 15.6;
+  const double step = pool->kda ? 2.0 : 2.5, extra = pool->kda ? 10.4 : 8.0, load = pool->kda ? .071 : 0.0;
   const int64_t C = pool->kda ? kc::C : pf::PC;
   int64_t longest = 0;
   for (int64_t b = 0; b < batch; b++) longest = cu[b + 1] - cu[b] > longest ? cu[b + 1] - cu[b] : longest;
-  double best = .85 * whole_chunk * (double)((longest + C - 1) / C);
+  double best = (pool->kda ? .97 : .85) * whole_chunk * (double)((longest + C - 1) / C);
   for (int64_t P = 2; P * H <= cus && P * C < longest + C; P++) {
     const int64_t L = ((longest + P - 1) / P + C - 1) / C * C;
     int64_t whole = 0, summaries = 0;
@@ -7008,7 +7013,7 @@ int sq_prefill_plan(const sq_pool *pool, const int32_t *cu, int64_t batch, int32
       summaries += n > 1 ? n - 1 : 0;
     }
     if (whole * H > cus || summaries * H > cus) break;
-    const double t = split_chunk * (double)(L / C) + step * (double)P + extra;
+    const double t = split_chunk * (double)(L / C) + step * (double)P + load * (double)(whole * H) + extra;
     if (t < best) {
       best = t;
       out->tokens = (int32_t)L;

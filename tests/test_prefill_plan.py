@@ -50,3 +50,10 @@ def test_split_arguments_are_checked():
         assert L.sq_prefill_split(pool, args, segments, None) == -22
     with pytest.raises(ValueError):
         N.check(L.sq_prefill_plan(pool, None, 1, CUS, N.PrefillSegments()), "plan")
+
+
+@pytest.mark.parametrize("tokens,split", [(256, False), (640, True)])
+@pytest.mark.parametrize("batch,heads", [(2, 32), (1, 64), (3, 16), (7, 8)])
+def test_short_kda_sequences_stay_whole(tokens, split, batch, heads):
+    """256 tokens in segments of 64 measured slower than whole, 640 tokens faster cut."""
+    assert bool(_plan([tokens] * batch, heads, "kda").tokens) is split
