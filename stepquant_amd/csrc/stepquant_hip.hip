@@ -6972,16 +6972,19 @@ int sq_create_cu_stream(int32_t device, int32_t cus, void **stream, int32_t *act
   return 0;
 }
 
+// compute units of the current device, 0 where it cannot be asked
+static int compute_units() {
+  int dev = 0, n = 0;
+  return hipGetDevice(&dev) == hipSuccess &&
+                 hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess
+             ? n
+             : 0;
+}
+
 int sq_prefill_plan(const sq_pool *pool, const int32_t *cu, int64_t batch, int32_t cus, sq_prefill_segments *out) {
   if (!pool || !cu || !out || batch < 0) return fail(SQ_EINVAL, "prefill plan: null argument or negative batch");
   *out = sq_prefill_segments{0, 0, 0, nullptr};
-  if (cus <= 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      return check_launch("prefill plan: device query");
-    cus = n;
-  }
+  if (cus <= 0 && (cus = compute_units()) <= 0) return check_launch("prefill plan: device query");
   const int64_t H = pool->heads;
   if (batch == 0 || H < 1 || batch * H > cus) return 0;
   // Time of a call whose workgroups all fit the device at once (one per
@@ -7133,7 +7136,7 @@ int sq_prefill_split(const sq_pool *pool, const sq_prefill_args *a, const sq_pre
   D.seg_trans = split ? D.seg_state + sg->workspace_bytes / (2 * sizeof(float)) : nullptr;
   const unsigned tiles = (unsigned)(a->batch * H), count = split ? (unsigned)sg->count : 1u;
   // longest sequences first when the workgroups (one per compute unit) do not all start at once
-  const bool ranked = !split && tiles > 256;
+  const bool ranked = !split && tiles > (unsigned)compute_units();
   const auto whole = pool->kda ? (ranked ? kc::kda_chunk_kernel<false, true> : kc::kda_chunk_kernel<false, false>)
                                : (ranked ? pf::prefill_kernel<false, true> : pf::prefill_kernel<false, false>);
   const auto summary = pool->kda ? kc::kda_chunk_kernel<true, false> : pf::prefill_kernel<true, false>;
