@@ -3351,7 +3351,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KDA128_WAVE
 // bytes, lane l receives byte l % 8 of rows l / 8 + 2 k), new carriers go
 // back as one LDS byte each (the low byte of 1.5 2^23 + z) in a padded
 // plane, and per-row constants are formed once per row instead of by each of
-// its 32 lanes.  Four workgroups per CU (128 registers, 28 KB of LDS).
+// its 32 lanes.  Four workgroups per CU (128 registers, 31 KB of LDS; at that
+// bound the GDN writer spills 8 values and the fused forms 2 to 20, the
+// readouts and the KDA writer none).
 // Bound by VALU issue and the dependent phases.  B = 128, 32 heads, GDN@6:
 // readout 30 us and writer 51 us; the general kernel (one LDS byte per value,
 // the tables and divisions in every lane) 74 and 147 us.
@@ -6043,13 +6045,13 @@ __global__ __launch_bounds__(256) void format_kernel(FmtDev F, StepDev S) {
 // its retention are formed once, not by each of its 32 lanes; codes are
 // rounded by the addition of 1.5 2^23 and packed W bits wide without
 // branches.  Four workgroups per CU (128 registers).  sym_int6, B = 256, 32
-// heads: 97 us a step, 219 us in format_kernel; bound by VALU issue.  FP32
-// pages of that size: 227 us, 290 us in format_kernel; bound by memory (1.07
-// GB read and written a step, 4.7 TB/s; a large copy reaches 4.9).
+// heads: 96 us a step, 219 us in format_kernel; bound by VALU issue.  FP32
+// pages of that size: 226 us, 290 us in format_kernel; bound by memory (1.07
+// GB read and written a step, 4.8 TB/s; a large copy reaches 4.9).
 // DSQ: the row means need each row's columns in a fixed order, so |x| passes
 // through LDS half the rows at a time, in the place of the codes, and 8
-// threads sum a row; 155 registers, three workgroups per CU (held to 128 it
-// spilled 37 values: 304 us).  dsq_int6, that size: 174 us, 430 us in
+// threads sum a row; 168 registers and 21 spilled values, three workgroups per
+// CU (held to 128 it spilled 37: 304 us).  dsq_int6, that size: 166-174 us, 430 us in
 // format_kernel; bound by VALU issue (two quotients a value).
 // =====================================================================
 namespace sym {
